@@ -135,20 +135,27 @@ void run_graph(hipStream_t s, GraphSlot* slots, const void* key, F&& body) {
 // (also for eigenvalues only), the own blocked back-transformation with the
 // reflectors.  Same outputs as syevd(): w ascending, A = eigenvectors.
 void syevd_own(hipStream_t s, rocblas_handle rb, bool vectors, int n, double*& A, double* w, double* E, double* tau,
-               double*& Z, double* work, double* owork, int* dinfo, hipEvent_t* tev = nullptr,
+               double*& Z, double* work, double* owork, int* dinfo, bool split, hipEvent_t* tev = nullptr,
                SolveGraphs* gr = nullptr) {
     if (tev) QK_HIP(hipEventRecord(tev[0], s));
     double* Ain = A;
-    auto trd = [&] { sytrd_upper(s, n, Ain, w, E, tau, work, 32); };
-    if (gr) run_graph(s, gr->trd, Ain, trd);
+    // Columns in registers wait inside the launch and are read back: never captured.
+    // Eigenvectors that go into a split-precision contraction (split) come from the
+    // launch-per-column form: the slices round by the vectors' last bits and signs,
+    // which differ between the two (2e-11 of a self-energy on the H50 lattice), and
+    // evGW's DIIS makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
+    int m = 0;
+    const bool resident = !(split && vectors) && trd_resident_fits(std::min(n, trd_resident_max())) && !stream_capturing(s);
+    auto trd = [&] { m = sytrd_upper(s, n, Ain, w, E, tau, work, 32, vectors ? owork : nullptr, resident); };
+    if (gr && !resident) run_graph(s, gr->trd, Ain, trd);
     else trd();
     if (tev) QK_HIP(hipEventRecord(tev[1], s));
     if (vectors) {
         rb_check(rocsolver_dstedc(rb, rocblas_evect_tridiagonal, n, w, E, Z, n, dinfo), "rocsolver_dstedc");
         if (tev) QK_HIP(hipEventRecord(tev[2], s));
         double* Zin = Z;
-        auto orm = [&] { ormtr_upper(s, n, Ain, tau, Zin, owork); };
-        if (gr) run_graph(s, gr->orm, Ain, orm);
+        auto orm = [&] { ormtr_upper(s, n, Ain, tau, Zin, owork, m); };
+        if (gr && m == (resident ? std::min(n, trd_resident_max()) : 0)) run_graph(s, gr->orm, Ain, orm);
         else orm();
         if (tev) QK_HIP(hipEventRecord(tev[3], s));
         std::swap(A, Z);
@@ -575,7 +582,7 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
         if (!done) {
             if (c->eig_mode & 2) {
                 syevd_own(c->s, c->rb, vectors, c->nS, c->Cm, c->Om, c->work, c->tau, c->Zev, c->trd_work,
-                          c->orm_work, c->info, c->ev3, &c->graphs);
+                          c->orm_work, c->info, c->precision != 0, c->ev3, &c->graphs);
                 float ms = 0.f;
                 QK_HIP(hipEventSynchronize(c->ev3[1]));
                 QK_HIP(hipEventElapsedTime(&ms, c->ev3[0], c->ev3[1]));

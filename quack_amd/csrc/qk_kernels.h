@@ -129,13 +129,33 @@ void gather_bov(hipStream_t s, const double* B, double* Bov, int naux, int n, in
 // Householder tridiagonalisation, upper triangle, LAPACK dsytrd layout (qk_sytrd.hip);
 // work holds sytrd_work_doubles(n, nb) doubles, nb <= 64.
 size_t sytrd_work_doubles(int n, int nb);
-void sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb);
-// Z <- Q Z with the reflectors sytrd_upper left in A, TAU (LAPACK dormtr,
-// SIDE = 'L', UPLO = 'U', TRANS = 'N'); work holds ormtr_work_doubles(n).
+// V (or null: none wanted): where ormtr_upper's work holds the reflectors.  With
+// resident, the last columns run in registers (qk_trdres.hip): no graph capture,
+// and one host wait.  Returns the order m of that part (0: none): its reflectors
+// are in V only, the others in A only.
+int sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, double* V,
+                bool resident);
+// Z <- Q Z with the reflectors sytrd_upper left in A, TAU and, columns before m - 1,
+// in work (LAPACK dormtr, SIDE = 'L', UPLO = 'U', TRANS = 'N'); work holds
+// ormtr_work_doubles(n) and starts with V.
 size_t ormtr_work_doubles(int n);
-void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work);
+void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work, int m);
 // A symmetric from its upper triangle: A[i, j] = A[j, i] for i > j
 void sym_lower(hipStream_t s, double* A, int n);
 void permute_cols(hipStream_t s, const double* X, const int* perm, double* out, int n);
+
+// Tridiagonalisation with the matrix in registers (qk_trdres.hip), the conventions of
+// sytrd_upper: order n <= trd_resident_max() (trd_resident_fits: on this device),
+// batch matrices sA apart, only the upper triangle of A is read and A is kept.  V
+// (or null): column j is reflector j with its unit element and zeros below it, rows
+// < n; D, E, TAU are sd apart; words: trd_resident_words(n, batch) doubles.  Returns
+// whether the launch can give up a wait: then the device word trd_resident_fail()
+// has to be read, and the outputs are void where it is set.
+int trd_resident_max();
+bool trd_resident_fits(int n);
+size_t trd_resident_words(int n, int batch);
+const int* trd_resident_fail(int n, int batch, const double* words);
+bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
+                  long long sV, double* D, double* E, double* TAU, long long sd, int batch, double* words);
 
 }  // namespace qk

@@ -492,8 +492,9 @@ __global__ void k_copy_v(const double* __restrict__ V, int n, int m, int nbp, do
 constexpr int OK = 128;   // reflectors per block
 constexpr int OKC = 512;  // rows per split-K chunk of V^T Z
 
-// V (n x nbk, zero-padded columns past n-1) and the padded taus
-__global__ void k_build_v(const double* __restrict__ A, int n, const double* __restrict__ TAU, int nbk,
+// V (n x nbk, zero-padded columns past n-1) and the padded taus; rows < m of the
+// columns before m - 1 are in V already
+__global__ void k_build_v(const double* __restrict__ A, int n, const double* __restrict__ TAU, int nbk, int m,
                           double* __restrict__ V, double* __restrict__ taup) {
     const long long total = (long long)n * nbk;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
@@ -501,7 +502,7 @@ __global__ void k_build_v(const double* __restrict__ A, int n, const double* __r
         const int r = (int)(t % n), j = (int)(t / n);
         double v = 0.0;
         if (j < n - 1) v = r < j ? A[r + (long long)n * (j + 1)] : (r == j ? 1.0 : 0.0);
-        V[t] = v;
+        if (j >= m - 1 || r >= m) V[t] = j < m - 1 ? 0.0 : v;
         if (r == 0) taup[j] = j < n - 1 ? TAU[j] : 0.0;
     }
 }
@@ -546,11 +547,15 @@ size_t sytrd_work_doubles(int n, int nb) {
     const size_t ntiles = (size_t)nt * (nt + 1) / 2;
     const size_t ng = groups_before(nt);
     const size_t nblk = (n + 63) / 64;
-    return 3 * (size_t)n * nb + (ntiles + ng) * TS + ng + 2 * (2 * (size_t)nb * nblk) + nblk + 8;
+    return 3 * (size_t)n * nb + (ntiles + ng) * TS + ng + 2 * (2 * (size_t)nb * nblk) + nblk + 8 +
+           trd_resident_words(std::min(n, trd_resident_max()), 1);
 }
 
-void sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb) {
-    QK_CHECK(n >= 1 && nb >= 1 && nb <= 64, QK_E_ARG, "sytrd: bad size");
+namespace {
+
+// columns c_hi down to c_end (>= 1), two launches each
+void sytrd_columns(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, int c_hi,
+                   int c_end) {
     const int nt_all = (n + TS - 1) / TS;
     const size_t ntiles_all = (size_t)nt_all * (nt_all + 1) / 2;
     const size_t ng_all = groups_before(nt_all);
@@ -566,9 +571,8 @@ void sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* 
     double* pnorm = tpart1 + 2 * (size_t)nb * nblk_all;
     double* scal = pnorm + nblk_all;  // two slots of (beta, tau, scale): [0..2] and [4..6]
     const int ldw = n, ldt = nblk_all;
-    int c_hi = n - 1;  // 0-based columns c_hi down to 1 carry reflectors
-    while (c_hi >= 1) {
-        const int nbp = std::min(nb, c_hi);
+    while (c_hi >= c_end) {
+        const int nbp = std::min(nb, c_hi - c_end + 1);
         const int c_lo = c_hi - nbp + 1;
         // first column of the panel: no panel terms; its norm partials and diagonal
         hipLaunchKernelGGL(k_col_update, dim3((c_hi + 1 + 63) / 64), dim3(TBW), 0, s, A, n, W, ldw, c_hi, 0, 0, -1,
@@ -607,10 +611,34 @@ void sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* 
         }
         c_hi = c_lo - 1;
     }
-    hipLaunchKernelGGL(k_d0, dim3(1), dim3(1), 0, s, A, D);
-    QK_HIP(hipGetLastError());
 }
 
+}  // namespace
+
+int sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, double* V,
+                bool resident) {
+    QK_CHECK(n >= 1 && nb >= 1 && nb <= 64, QK_E_ARG, "sytrd: bad size");
+    // 0-based columns n-1 down to 1 carry reflectors.  Those of the leading block
+    // that fits the registers run there: at n = 1326 8.9 ms instead of 22.
+    const int m = std::min(n, trd_resident_max());
+    if (resident && trd_resident_fits(m)) {
+        sytrd_columns(s, n, A, D, E, TAU, work, nb, n - 1, m);
+        double* words = work + sytrd_work_doubles(n, nb) - trd_resident_words(m, 1);
+        int fail = 0;
+        if (trd_resident(s, m, A, n, 0, V, n, 0, D, E, TAU, 0, 1, words)) {
+            QK_HIP(hipMemcpyAsync(&fail, trd_resident_fail(m, 1, words), sizeof(int), hipMemcpyDeviceToHost, s));
+            QK_HIP(hipStreamSynchronize(s));
+        }
+        if (!fail) return m;
+        // another process's launch shares the device: A still holds the block
+        sytrd_columns(s, n, A, D, E, TAU, work, nb, m - 1, 1);
+    } else {
+        sytrd_columns(s, n, A, D, E, TAU, work, nb, n - 1, 1);
+    }
+    hipLaunchKernelGGL(k_d0, dim3(1), dim3(1), 0, s, A, D);
+    QK_HIP(hipGetLastError());
+    return 0;
+}
 
 size_t ormtr_work_doubles(int n) {
     const int nblk = (n - 1 + OK - 1) / OK;
@@ -620,7 +648,7 @@ size_t ormtr_work_doubles(int n) {
            (size_t)OK * n;
 }
 
-void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work) {
+void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work, int m) {
     QK_CHECK(n >= 1, QK_E_ARG, "ormtr: bad size");
     if (n == 1) return;
     const int nblk = (n - 1 + OK - 1) / OK;
@@ -634,7 +662,7 @@ void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, doubl
     double* W2 = W1p + (size_t)oks * OK * n;            // OK x n
     const long long tot = (long long)n * nbk;
     hipLaunchKernelGGL(k_build_v, dim3((unsigned)std::min<long long>((tot + 255) / 256, 65536)), dim3(256), 0, s, A,
-                       n, TAU, nbk, V, taup);
+                       n, TAU, nbk, m, V, taup);
     QK_HIP(hipGetLastError());
     {
         Batch bg;

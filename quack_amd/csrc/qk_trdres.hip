@@ -1,0 +1,577 @@
+// Householder tridiagonalisation with the matrix held in registers (gfx950).
+//
+// Same result as sytrd_upper (qk_sytrd.hip; LAPACK dsytd2, UPLO = 'U'), for
+// matrices of order n <= TRD_MAX and for the leading TRD_MAX x TRD_MAX part
+// that is left of a larger one.  The launch-per-step form pays two launches
+// a column (about 16 us a column at n = 1326, whatever the work); here one
+// launch runs every column and the G workgroups that share a matrix meet once
+// a column.
+//
+// Layout.  Workgroup g owns the full rows r = g (mod G), so y = A v needs no
+// sum over workgroups, and the rows that are still active stay balanced as the
+// matrix shrinks.  At column c every workgroup
+//   1. applies the previous column's A -= v w^T + w v^T to its rows and forms
+//      y_r = A_r v in the same pass over its registers;
+//   2. publishes its y_r; the owner of row c-1 publishes that row as well;
+//   3. reads all of y and row c-1, and from them computes w and the next
+//      column x = A(:, c-1) - v w_{c-1} - w and its reflector.  Every workgroup
+//      does the same arithmetic in the same order, so all hold the same bits
+//      and no second exchange is needed.
+// The exchange carries its own arrival flags: each double travels as two 64-bit
+// words, half of the value beside the column number, stored and loaded with
+// single agent-scope atomics, so a reader that sees the column number has the
+// value (one trip through the shared cache instead of store, counter, poll and
+// load).  Two buffers alternate: a workgroup can write column c-2 only after
+// it has read every workgroup's column c-1, which they publish after reading c.
+//
+// Two shapes of the same algorithm: k_trd_small (n <= 512) gives each wave its
+// own rows and all columns, so every sum over columns stays inside a wave and
+// a column costs one barrier; k_trd_wide (n <= 3072) spreads the columns over
+// the workgroup's 512 threads.
+//
+// Bound: the exchange and the barriers of a column, not arithmetic or memory.
+// Measured per column: 1.4 us at n = 64, 2.5 at 160 (one workgroup), 3.3 at 225,
+// 3.6 at 324, 6.2 at 900, 6.8 at 1326, 7.5 at 2025, 8.1 at 3072; 24 matrices of 324
+// take 1.22 ms together, one 1.17.
+//
+// Waits end: a reader that sees no progress for SPIN_TICKS raises *fail, which
+// the other workgroups read, and all leave; the caller then runs sytrd_upper.
+// Launches whose workgroups wait for each other are kept one after another on
+// the device (resident_gate), each with at most one workgroup per CU.
+#include <mutex>
+
+#include "qk_kernels.h"
+
+namespace qk {
+namespace {
+
+typedef unsigned long long u64;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int TT = 512;  // threads per workgroup: two waves per SIMD, 256 VGPRs each
+constexpr long long SPIN_TICKS = 200000000LL;  // 2 s of the 100 MHz clock
+
+__device__ inline void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int CTRL>
+__device__ inline double row_rot(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// sum over the 16 lanes of a row, in every lane of it
+__device__ inline double row_sum(double v) {
+    v += row_rot<0x128>(v);
+    v += row_rot<0x124>(v);
+    v += row_rot<0x122>(v);
+    v += row_rot<0x121>(v);
+    return v;
+}
+// v_permlane32_swap / v_permlane16_swap of two doubles, then their sum: the upper
+// half (odd rows) of a changes places with the lower half (even rows) of b
+__device__ inline double swap32_add(double a, double b) {
+    const u32x2 l = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const u32x2 h = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+__device__ inline double swap16_add(double a, double b) {
+    const u32x2 l = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const u32x2 h = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+// sum over the wave, in every lane
+__device__ inline double wave_sum(double v) {
+    v = row_sum(v);
+    v = swap16_add(v, v);
+    return swap32_add(v, v);
+}
+// four wave sums at once: lanes of row q (16 lanes) get the sum of a[q]
+__device__ inline double wave_sum4(const double* a) {
+    const double s0 = swap32_add(a[0], a[2]), s1 = swap32_add(a[1], a[3]);
+    return row_sum(swap16_add(s0, s1));
+}
+__device__ inline double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// one double with its column number beside either half
+__device__ inline void publish(u64* w, double v, unsigned tag) {
+    const u64 t = (u64)tag << 32;
+    __hip_atomic_store(w, t | (unsigned)__double2loint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w + 1, t | (unsigned)__double2hiint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool arrived(const u64* w, unsigned tag, double& v) {
+    const u64 a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const u64 b = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __hiloint2double((int)(unsigned)b, (int)(unsigned)a);
+    return (unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag;
+}
+// bookkeeping of a wait; true when it has to be given up
+__device__ inline bool give_up(unsigned& spins, long long& t0, int* fail) {
+    if ((++spins & 255) != 0) return false;
+    if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return true;
+    const long long t = wall_clock64();
+    if (t0 == 0) t0 = t;
+    if (t - t0 < SPIN_TICKS) return false;
+    __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+struct TrdArgs {
+    const double* A;  // upper triangle read
+    long long lda, sA;
+    int n, G;
+    double* V;  // reflectors, v_j in column j (rows < n), or null
+    long long ldv, sV;
+    double *D, *E, *TAU;
+    long long sd;  // stride of D, E, TAU between matrices
+    u64* X;        // exchange words, 8 n per matrix, zeroed
+    int* fail;
+};
+
+__device__ inline double load_sym(const double* A, long long lda, int r, int col) {
+    return col <= r ? A[col + lda * r] : A[r + lda * col];
+}
+
+struct Reflector {
+    double beta, tau, scale;
+};
+__device__ inline Reflector reflector(double alpha, double xx) {
+    Reflector h;
+    if (xx == 0.0) {
+        h.beta = alpha;
+        h.tau = 0.0;
+        h.scale = 0.0;
+    } else {
+        const double nrm = sqrt(alpha * alpha + xx);
+        h.beta = alpha >= 0.0 ? -nrm : nrm;
+        h.tau = (h.beta - alpha) / h.beta;
+        h.scale = 1.0 / (alpha - h.beta);
+    }
+    return h;
+}
+
+// n <= 64 KC <= 512.  Wave q of workgroup g owns rows g + G (q + 8 j), j < R; lane l
+// holds columns l + 64 k of them.  Needs n <= 8 R G.
+template <int KC, int R>
+__global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
+    static_assert(R % 4 == 0 && KC <= 8, "rows go in fours; one column a thread in the exchange");
+    __shared__ double ys[2][64 * KC], as[2][64 * KC];
+    __shared__ double vw[8][2][64 * KC];  // each wave's copy of v and w, for its rows' entries
+    __shared__ int quit;
+    const int G = p.G, z = blockIdx.x / G, g = blockIdx.x % G, n = p.n;
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const double* A = p.A + z * p.sA;
+    double* V = p.V ? p.V + z * p.sV : nullptr;
+    double *D = p.D + z * p.sd, *E = p.E + z * p.sd, *TAU = p.TAU + z * p.sd;
+    u64* X = p.X + (long long)z * 8 * n;
+    const bool writer = g == 0 && q == 0;
+    double* vq = vw[q][0];
+    double* wq = vw[q][1];
+    double a[R][KC], v[KC], vp[KC], wp[KC], x[KC];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int r = g + G * (q + 8 * j);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = lane + 64 * k;
+            a[j][k] = r < n && col < n ? load_sym(A, p.lda, r, col) : 0.0;
+        }
+    }
+    int c = n - 1;
+    double xx = 0.0, alpha = 0.0;
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+        const int col = lane + 64 * k;
+        x[k] = col <= c ? A[col + p.lda * c] : 0.0;
+        vp[k] = wp[k] = 0.0;
+        vq[col] = wq[col] = 0.0;
+        if (writer && col == c) D[c] = x[k];
+    }
+    if (threadIdx.x == 0) quit = 0;
+    lds_barrier();
+    unsigned spins = 0;
+    for (; c >= 1; --c) {
+        const int par = c & 1;
+        // reflector of column c from x
+        xx = 0.0;
+        double sel = 0.0;
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = lane + 64 * k;
+            if (k == (c - 1) >> 6) sel = x[k];
+            if (col < c - 1) xx += x[k] * x[k];
+        }
+        alpha = lane_value(sel, (c - 1) & 63);
+        const Reflector h = reflector(alpha, wave_sum(xx));
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = lane + 64 * k;
+            v[k] = col < c - 1 ? x[k] * h.scale : (col == c - 1 ? 1.0 : 0.0);
+        }
+        // update of the previous column and y = A v, row by row
+#pragma unroll
+        for (int j0 = 0; j0 < R; j0 += 4) {
+            if (g + G * (q + 8 * j0) < c) {
+                double acc[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int r = g + G * (q + 8 * (j0 + u));
+                    acc[u] = 0.0;
+                    if (r < c) {
+                        const double vr = vq[r], wr = wq[r];
+#pragma unroll
+                        for (int k = 0; k < KC; ++k) {
+                            const double t = a[j0 + u][k] - vr * wp[k] - wr * vp[k];
+                            a[j0 + u][k] = t;
+                            acc[u] += t * v[k];
+                        }
+                        if (r == c - 1) {  // this row goes to everyone
+#pragma unroll
+                            for (int k = 0; k < KC; ++k) {
+                                const int col = lane + 64 * k;
+                                if (col < c) {
+                                    if (G > 1) publish(X + 4LL * n * par + 2LL * n + 2 * col, a[j0 + u][k], c);
+                                    else as[par][col] = a[j0 + u][k];
+                                }
+                            }
+                        }
+                    }
+                }
+                const double y = wave_sum4(acc);
+                const int r = g + G * (q + 8 * (j0 + (lane >> 4)));
+                if ((lane & 15) == 0 && r < c) {
+                    if (G > 1) publish(X + 4LL * n * par + 2 * r, y, c);
+                    else ys[par][r] = y;
+                }
+            }
+        }
+        if (V && g == c % G && q == ((c / G) & 7)) {
+#pragma unroll
+            for (int k = 0; k < KC; ++k) {
+                const int col = lane + 64 * k;
+                if (col < n) V[col + p.ldv * (c - 1)] = v[k];
+            }
+        }
+        if (writer && lane == 0) {
+            E[c - 1] = h.beta;
+            TAU[c - 1] = h.tau;
+        }
+        if (G > 1 && (int)threadIdx.x < c) {
+            const u64* w = X + 4LL * n * par + 2 * threadIdx.x;
+            double y = 0.0, ao = 0.0;
+            long long t0 = 0;
+            for (;;) {
+                const bool f1 = arrived(w, c, y), f2 = arrived(w + 2LL * n, c, ao);
+                if (f1 && f2) break;
+                if (give_up(spins, t0, p.fail)) {
+                    quit = 1;
+                    break;
+                }
+            }
+            ys[par][threadIdx.x] = y;
+            as[par][threadIdx.x] = ao;
+        }
+        lds_barrier();
+        if (G > 1 && quit) return;
+        // w = tau y - tau^2 (y . v) v / 2
+        double y[KC], dot = 0.0;
+        sel = 0.0;
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = lane + 64 * k;
+            y[k] = col < c ? ys[par][col] : 0.0;
+            x[k] = col < c ? as[par][col] : 0.0;
+            dot += y[k] * v[k];
+        }
+        const double half = -0.5 * h.tau * h.tau * wave_sum(dot);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            wp[k] = h.tau * y[k] + half * v[k];
+            vp[k] = v[k];
+            if (k == (c - 1) >> 6) sel = wp[k];
+        }
+        const double wl = lane_value(sel, (c - 1) & 63);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = lane + 64 * k;
+            x[k] = col < c ? x[k] - (v[k] * wl + wp[k]) : 0.0;  // v(c-1) = 1
+            if (writer && col == c - 1) D[c - 1] = x[k];
+            vq[col] = v[k];
+            wq[col] = wp[k];
+        }
+    }
+}
+
+// n <= 512 KC.  Workgroup g owns rows g + G j, j < R; thread t holds columns t + 512 k
+// of them.  Needs n <= R G.
+template <int KC, int R>
+__global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
+    static_assert(R % 4 == 0 && R <= 64, "rows go in fours");
+    __shared__ double vs[TT * KC], ws[TT * KC];
+    __shared__ double yp[8][R];
+    __shared__ double red1[8], red2[8];
+    __shared__ double ylast, xlast;
+    __shared__ int quit;
+    const int G = p.G, z = blockIdx.x / G, g = blockIdx.x % G, n = p.n;
+    const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
+    const double* A = p.A + z * p.sA;
+    double* V = p.V ? p.V + z * p.sV : nullptr;
+    double *D = p.D + z * p.sd, *E = p.E + z * p.sd, *TAU = p.TAU + z * p.sd;
+    u64* X = p.X + (long long)z * 8 * n;
+    double a[R][KC], v[KC], vp[KC], wp[KC], x[KC];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int r = g + G * j;
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = tid + TT * k;
+            a[j][k] = r < n && col < n ? load_sym(A, p.lda, r, col) : 0.0;
+        }
+    }
+    int c = n - 1;
+    double part = 0.0;
+#pragma unroll
+    for (int k = 0; k < KC; ++k) {
+        const int col = tid + TT * k;
+        x[k] = col <= c ? A[col + p.lda * c] : 0.0;
+        vp[k] = wp[k] = 0.0;
+        vs[col] = ws[col] = 0.0;
+        if (g == 0 && col == c) D[c] = x[k];
+        if (col < c - 1) part += x[k] * x[k];
+        if (col == c - 1) xlast = x[k];
+    }
+    part = wave_sum(part);
+    if (lane == 0) red2[q] = part;
+    if (tid == 0) quit = 0;
+    lds_barrier();
+    unsigned spins = 0;
+    for (; c >= 1; --c) {
+        const int par = c & 1;
+        double xx = 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) xx += red2[u];
+        const Reflector h = reflector(xlast, xx);
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = tid + TT * k;
+            v[k] = col < c - 1 ? x[k] * h.scale : (col == c - 1 ? 1.0 : 0.0);
+        }
+#pragma unroll
+        for (int j0 = 0; j0 < R; j0 += 4) {
+            if (g + G * j0 < c) {
+                double acc[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int r = g + G * (j0 + u);
+                    acc[u] = 0.0;
+                    if (r < c) {
+                        const double vr = vs[r], wr = ws[r];
+#pragma unroll
+                        for (int k = 0; k < KC; ++k)
+                            if (TT * k < c) {
+                                const double t = a[j0 + u][k] - vr * wp[k] - wr * vp[k];
+                                a[j0 + u][k] = t;
+                                acc[u] += t * v[k];
+                            }
+                        if (r == c - 1) {
+#pragma unroll
+                            for (int k = 0; k < KC; ++k) {
+                                const int col = tid + TT * k;
+                                if (col < c) publish(X + 4LL * n * par + 2LL * n + 2 * col, a[j0 + u][k], c);
+                            }
+                        }
+                    }
+                }
+                const double y = wave_sum4(acc);
+                if ((lane & 15) == 0) yp[q][j0 + (lane >> 4)] = y;
+            }
+        }
+        lds_barrier();
+        if (tid < R) {
+            const int r = g + G * tid;
+            if (r < c) {
+                double y = 0.0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) y += yp[u][tid];
+                publish(X + 4LL * n * par + 2 * r, y, c);
+            }
+        }
+        if (V && g == c % G) {
+#pragma unroll
+            for (int k = 0; k < KC; ++k) {
+                const int col = tid + TT * k;
+                if (col < n) V[col + p.ldv * (c - 1)] = v[k];
+            }
+        }
+        if (g == 0 && tid == 0) {
+            E[c - 1] = h.beta;
+            TAU[c - 1] = h.tau;
+        }
+        double y[KC], dot = 0.0;
+        {
+            long long t0 = 0;
+            for (;;) {
+                bool all = true;
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    const int col = tid + TT * k;
+                    y[k] = x[k] = 0.0;
+                    if (col < c) {
+                        const u64* w = X + 4LL * n * par + 2 * col;
+                        const bool f1 = arrived(w, c, y[k]), f2 = arrived(w + 2LL * n, c, x[k]);
+                        all = all && f1 && f2;
+                    }
+                }
+                if (all) break;
+                if (give_up(spins, t0, p.fail)) {
+                    quit = 1;
+                    break;
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            dot += y[k] * v[k];
+            if (tid + TT * k == c - 1) ylast = y[k];
+        }
+        dot = wave_sum(dot);
+        if (lane == 0) red1[q] = dot;
+        lds_barrier();
+        if (quit) return;
+        dot = 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) dot += red1[u];
+        const double half = -0.5 * h.tau * h.tau * dot;
+        const double wl = h.tau * ylast + half;  // w(c-1), v(c-1) = 1
+        part = 0.0;
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int col = tid + TT * k;
+            wp[k] = h.tau * y[k] + half * v[k];
+            vp[k] = v[k];
+            x[k] = col < c ? x[k] - (v[k] * wl + wp[k]) : 0.0;
+            if (g == 0 && col == c - 1) D[c - 1] = x[k];
+            vs[col] = v[k];
+            ws[col] = wp[k];
+            if (col < c - 2) part += x[k] * x[k];
+            if (col == c - 2) xlast = x[k];
+        }
+        part = wave_sum(part);
+        if (lane == 0) red2[q] = part;
+        lds_barrier();
+    }
+}
+
+__global__ void k_zero_words(u64* __restrict__ X, long long count) {
+    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < count; t += (long long)gridDim.x * blockDim.x)
+        X[t] = 0;
+}
+
+// The kernels above wait inside a launch for the other workgroups of the same
+// launch, so two such launches must not each hold a part of the device: every
+// one waits for the one before it, on whatever stream that ran.
+struct Gate {
+    std::mutex mu;
+    hipEvent_t last[64] = {};
+};
+Gate& gate() {
+    static Gate* g = new Gate();  // lives until process exit, as the streams that wait on its events may
+    return *g;
+}
+template <class F>
+void resident_gate(hipStream_t s, F&& launch) {
+    int dev = 0;
+    QK_HIP(hipGetDevice(&dev));
+    QK_CHECK(dev >= 0 && dev < 64, QK_E_HIP, "device number");
+    Gate& g = gate();
+    std::lock_guard<std::mutex> lock(g.mu);
+    if (g.last[dev]) QK_HIP(hipStreamWaitEvent(s, g.last[dev], 0));
+    else QK_HIP(hipEventCreateWithFlags(&g.last[dev], hipEventDisableTiming));
+    launch();
+    QK_HIP(hipGetLastError());
+    QK_HIP(hipEventRecord(g.last[dev], s));
+}
+
+int compute_units() {
+    int dev = 0, cu = 0;
+    QK_HIP(hipGetDevice(&dev));
+    QK_HIP(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
+    return cu;
+}
+
+// Workgroups per matrix.  R KC registers pairs hold a thread's share of A (at most 72
+// of the 128 pairs; the rest are the column vectors).  n <= 160 fits one
+// workgroup, which needs no exchange at all.
+struct Shape {
+    int kc, r, g;
+};
+Shape trd_shape(int n) {
+    if (n <= 64) return {1, 8, 1};
+    if (n <= 128) return {2, 16, 1};
+    if (n <= 160) return {3, 20, 1};
+    if (n <= 192) return {3, 12, 2};
+    if (n <= 256) return {4, 16, (n + 127) / 128};
+    if (n <= 384) return {6, 8, (n + 63) / 64};
+    if (n <= 512) return {8, 8, (n + 63) / 64};
+    if (n <= 1024) return {2, 32, (n + 31) / 32};
+    if (n <= 1536) return {3, 24, (n + 23) / 24};
+    if (n <= 2048) return {4, 16, (n + 15) / 16};
+    if (n <= 2560) return {5, 16, (n + 15) / 16};
+    return {6, 12, (n + 11) / 12};
+}
+
+}  // namespace
+
+int trd_resident_max() { return 3072; }
+size_t trd_resident_words(int n, int batch) { return 8 * (size_t)n * batch + 1; }
+const int* trd_resident_fail(int n, int batch, const double* words) {
+    return reinterpret_cast<const int*>(words + trd_resident_words(n, batch) - 1);
+}
+bool trd_resident_fits(int n) { return n >= 1 && n <= trd_resident_max() && trd_shape(n).g <= compute_units(); }
+
+bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
+                  long long sV, double* D, double* E, double* TAU, long long sd, int batch, double* words) {
+    QK_CHECK(trd_resident_fits(n) && lda >= n && (!V || ldv >= n) && batch >= 1, QK_E_ARG, "trd_resident: bad size");
+    const Shape sh = trd_shape(n);
+    u64* X = reinterpret_cast<u64*>(words);  // exchange words, then the flag of a wait given up
+    int* fail = reinterpret_cast<int*>(words + trd_resident_words(n, batch) - 1);
+    const int per = sh.g > 1 ? std::max(1, compute_units() / sh.g) : batch;  // matrices of one launch
+    if (sh.g > 1) {
+        const long long cnt = (long long)trd_resident_words(n, batch);
+        hipLaunchKernelGGL(k_zero_words, dim3((unsigned)std::min<long long>((cnt + 255) / 256, 1024)), dim3(256), 0, s, X,
+                           cnt);
+        QK_HIP(hipGetLastError());
+    }
+    for (int b0 = 0; b0 < batch; b0 += per) {
+        const int nb = std::min(per, batch - b0);
+        TrdArgs p{A + b0 * sA, lda, sA, n, sh.g, V ? V + b0 * sV : nullptr, ldv, sV, D + b0 * sd, E + b0 * sd,
+                  TAU + b0 * sd, sd, X + 8LL * n * b0, fail};
+        const dim3 grid(sh.g * nb), blk(TT);
+        auto go = [&] {
+            if (n <= 64) hipLaunchKernelGGL((k_trd_small<1, 8>), grid, blk, 0, s, p);
+            else if (n <= 128) hipLaunchKernelGGL((k_trd_small<2, 16>), grid, blk, 0, s, p);
+            else if (n <= 160) hipLaunchKernelGGL((k_trd_small<3, 20>), grid, blk, 0, s, p);
+            else if (n <= 192) hipLaunchKernelGGL((k_trd_small<3, 12>), grid, blk, 0, s, p);
+            else if (n <= 256) hipLaunchKernelGGL((k_trd_small<4, 16>), grid, blk, 0, s, p);
+            else if (n <= 384) hipLaunchKernelGGL((k_trd_small<6, 8>), grid, blk, 0, s, p);
+            else if (n <= 512) hipLaunchKernelGGL((k_trd_small<8, 8>), grid, blk, 0, s, p);
+            else if (n <= 1024) hipLaunchKernelGGL((k_trd_wide<2, 32>), grid, blk, 0, s, p);
+            else if (n <= 1536) hipLaunchKernelGGL((k_trd_wide<3, 24>), grid, blk, 0, s, p);
+            else if (n <= 2048) hipLaunchKernelGGL((k_trd_wide<4, 16>), grid, blk, 0, s, p);
+            else if (n <= 2560) hipLaunchKernelGGL((k_trd_wide<5, 16>), grid, blk, 0, s, p);
+            else hipLaunchKernelGGL((k_trd_wide<6, 12>), grid, blk, 0, s, p);
+        };
+        if (sh.g > 1) resident_gate(s, go);
+        else go();
+        QK_HIP(hipGetLastError());
+    }
+    return sh.g > 1;
+}
+
+}  // namespace qk
