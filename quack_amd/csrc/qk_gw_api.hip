@@ -130,40 +130,22 @@ void run_graph(hipStream_t s, GraphSlot* slots, const void* key, F&& body) {
     QK_HIP(hipGraphLaunch(ex, s));
 }
 
-// Full eigen-decomposition without dsyevd: own Householder tridiagonalisation
-// (qk_sytrd.hip), rocSOLVER's divide-and-conquer dstedc on the tridiagonal
-// (also for eigenvalues only), the own blocked back-transformation with the
-// reflectors.  Same outputs as syevd(): w ascending, A = eigenvectors.
-void syevd_own(hipStream_t s, rocblas_handle rb, bool vectors, int n, double*& A, double* w, double* E, double* tau,
-               double*& Z, double* work, double* owork, int* dinfo, bool split, hipEvent_t* tev = nullptr,
-               SolveGraphs* gr = nullptr) {
-    if (tev) QK_HIP(hipEventRecord(tev[0], s));
+// Full eigen-decomposition for a split-precision contraction (modes 2 and 3): the
+// launch-per-column tridiagonalisation (qk_sytrd.hip), rocSOLVER's dstedc, the
+// blocked back-transformation by GEMMs.  Same outputs as syevd(): w ascending,
+// A = eigenvectors.
+void syevd_own(hipStream_t s, rocblas_handle rb, int n, double*& A, double* w, double* E, double* tau, double*& Z,
+               double* work, double* owork, int* dinfo, hipEvent_t* tev, SolveGraphs* gr) {
+    QK_HIP(hipEventRecord(tev[0], s));
     double* Ain = A;
-    // Columns in registers wait inside the launch and are read back: never captured.
-    // Eigenvectors that go into a split-precision contraction (split) come from the
-    // launch-per-column form: the slices round by the vectors' last bits and signs,
-    // which differ between the two (2e-11 of a self-energy on the H50 lattice), and
-    // evGW's DIIS makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
-    int m = 0;
-    const bool resident = !(split && vectors) && trd_resident_fits(std::min(n, trd_resident_max())) && !stream_capturing(s);
-    auto trd = [&] { m = sytrd_upper(s, n, Ain, w, E, tau, work, 32, vectors ? owork : nullptr, resident); };
-    if (gr && !resident) run_graph(s, gr->trd, Ain, trd);
-    else trd();
-    if (tev) QK_HIP(hipEventRecord(tev[1], s));
-    if (vectors) {
-        rb_check(rocsolver_dstedc(rb, rocblas_evect_tridiagonal, n, w, E, Z, n, dinfo), "rocsolver_dstedc");
-        if (tev) QK_HIP(hipEventRecord(tev[2], s));
-        double* Zin = Z;
-        auto orm = [&] { ormtr_upper(s, n, Ain, tau, Zin, owork, m); };
-        if (gr && m == (resident ? std::min(n, trd_resident_max()) : 0)) run_graph(s, gr->orm, Ain, orm);
-        else orm();
-        if (tev) QK_HIP(hipEventRecord(tev[3], s));
-        std::swap(A, Z);
-    } else {
-        // eigenvalues only: divide-and-conquer into the spare matrix (rocSOLVER's
-        // dsterf, a sequential QL sweep, takes seconds at n ~ 5000)
-        rb_check(rocsolver_dstedc(rb, rocblas_evect_tridiagonal, n, w, E, Z, n, dinfo), "rocsolver_dstedc");
-    }
+    run_graph(s, gr->trd, Ain, [&] { sytrd_upper(s, n, Ain, w, E, tau, work, 32, nullptr, false); });
+    QK_HIP(hipEventRecord(tev[1], s));
+    rb_check(rocsolver_dstedc(rb, rocblas_evect_tridiagonal, n, w, E, Z, n, dinfo), "rocsolver_dstedc");
+    QK_HIP(hipEventRecord(tev[2], s));
+    double* Zin = Z;
+    run_graph(s, gr->orm, Ain, [&] { ormtr_upper(s, n, Ain, tau, Zin, owork); });
+    QK_HIP(hipEventRecord(tev[3], s));
+    std::swap(A, Z);
     int info = 0;
     QK_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
     QK_HIP(hipStreamSynchronize(s));
@@ -556,6 +538,36 @@ bool refine_eig(Ctx* c) {
 // Cm = eigenvectors (scaled to W when vectors), Om = excitation energies.
 int n_energies(const Ctx* c) { return c->nOb >= 0 ? 2 * c->nOrb : c->nOrb; }
 
+// The full solve of Cm: eigenvalues to Om, with vectors the eigenvectors in Cm's place.
+void solve_full(Ctx* c, bool vectors) {
+    const size_t need = eigh_work_doubles(c->nS, 1, vectors);
+    if (c->eigw_doubles < need) {
+        dfree(c->eigw);
+        c->eigw_doubles = 0;
+        c->eigw = dalloc<double>(need);
+        c->eigw_doubles = need;
+    }
+    eigh(c->s, c->nS, 1, c->Cm, (long long)c->nS * c->nS, c->Om, c->nS, vectors, c->eigw, c->info,
+         c->eig_mode & 2 ? c->ev3 : nullptr);
+    int info = 0;
+    QK_HIP(hipMemcpyAsync(&info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->s));
+    QK_HIP(hipStreamSynchronize(c->s));
+    QK_CHECK(info == 0, QK_E_EIG, "eigensolver: the matrix has entries that are not finite");
+}
+
+// The same for eigenvectors of a split-precision contraction, modes 2 and 3.
+void solve_split(Ctx* c) {
+    if (!c->Zev) {
+        const size_t S = c->nS;
+        c->Zev = dalloc<double>(S * S);
+        c->tau = dalloc<double>(S);
+        c->trd_work = dalloc<double>(sytrd_work_doubles(c->nS, 32));
+        c->orm_work = dalloc<double>(ormtr_work_doubles(c->nS));
+    }
+    syevd_own(c->s, c->rb, c->nS, c->Cm, c->Om, c->work, c->tau, c->Zev, c->trd_work, c->orm_work, c->info, c->ev3,
+              &c->graphs);
+}
+
 void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors) {
     {
         Stage st(c, 0);
@@ -580,24 +592,31 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
             ++c->eig_count[done ? 1 : 3];
         }
         if (!done) {
-            if (c->eig_mode & 2) {
-                syevd_own(c->s, c->rb, vectors, c->nS, c->Cm, c->Om, c->work, c->tau, c->Zev, c->trd_work,
-                          c->orm_work, c->info, c->precision != 0, c->ev3, &c->graphs);
-                float ms = 0.f;
-                QK_HIP(hipEventSynchronize(c->ev3[1]));
-                QK_HIP(hipEventElapsedTime(&ms, c->ev3[0], c->ev3[1]));
-                c->t_trd_total += ms;
-                c->n_trd_total += 1.0;
-                if (vectors) {
-                    QK_HIP(hipEventSynchronize(c->ev3[3]));
-                    QK_HIP(hipEventElapsedTime(&ms, c->ev3[1], c->ev3[2]));
-                    c->t_stedc_total += ms;
-                    QK_HIP(hipEventElapsedTime(&ms, c->ev3[2], c->ev3[3]));
-                    c->t_ormtr_total += ms;
-                }
-                ++c->eig_count[8];
+            // Eigenvectors that go into a split-precision contraction keep the solver they
+            // had: the slices round by the vectors' last bits and signs, which differ from
+            // solver to solver (2e-11 of a self-energy on the H50 lattice), and evGW's DIIS
+            // makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
+            const bool split = c->precision != 0 && vectors;
+            if (split && !(c->eig_mode & 2)) {
+                syevd(c->s, c->rb, true, c->nS, c->Cm, c->Om, c->work, c->info);
             } else {
-                syevd(c->s, c->rb, vectors, c->nS, c->Cm, c->Om, c->work, c->info);
+                if (split) solve_split(c);
+                else solve_full(c, vectors);
+                if (c->eig_mode & 2) {
+                    float ms = 0.f;
+                    QK_HIP(hipEventSynchronize(c->ev3[1]));
+                    QK_HIP(hipEventElapsedTime(&ms, c->ev3[0], c->ev3[1]));
+                    c->t_trd_total += ms;
+                    c->n_trd_total += 1.0;
+                    if (vectors) {
+                        QK_HIP(hipEventSynchronize(c->ev3[3]));
+                        QK_HIP(hipEventElapsedTime(&ms, c->ev3[1], c->ev3[2]));
+                        c->t_stedc_total += ms;
+                        QK_HIP(hipEventElapsedTime(&ms, c->ev3[2], c->ev3[3]));
+                        c->t_ormtr_total += ms;
+                    }
+                    ++c->eig_count[8];
+                }
             }
             ++c->eig_count[0];
             if ((c->eig_mode & 1) && vectors)
@@ -910,7 +929,7 @@ void release(Ctx* c) {
     int* is[] = {c->nit, c->done, c->info, c->active};
     for (int* p : is)
         if (p) (void)hipFree(p);
-    for (double* p : {c->Xv, c->Ym, c->Sm, c->Gm, c->lam, c->eig_dbuf, c->Zev, c->tau, c->trd_work, c->orm_work})
+    for (double* p : {c->Xv, c->Ym, c->Sm, c->Gm, c->lam, c->eig_dbuf, c->Zev, c->tau, c->trd_work, c->orm_work, c->eigw})
         if (p) (void)hipFree(p);
     for (int* p : {c->perm, c->eig_ibuf})
         if (p) (void)hipFree(p);
@@ -1222,13 +1241,6 @@ int qk_gw_set_precision(qk_gw_handle c, int mode) {
 int qk_gw_set_eigensolver(qk_gw_handle c, int mode, double de_max) {
     if (!c || mode < 0 || mode > 3 || !(de_max >= 0.0)) return QK_E_ARG;
     return guarded(&c->err, [&] {
-        if ((mode & 2) && !c->Zev) {
-            size_t S = c->nS;
-            c->Zev = dalloc<double>(S * S);
-            c->tau = dalloc<double>(S);
-            c->trd_work = dalloc<double>(sytrd_work_doubles(c->nS, 32));
-            c->orm_work = dalloc<double>(ormtr_work_doubles(c->nS));
-        }
         if ((mode & 1) && !c->Xv) {
             size_t S = c->nS;
             c->Xv = dalloc<double>(S * S);

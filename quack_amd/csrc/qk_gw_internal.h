@@ -136,12 +136,14 @@ struct qk_gw_ctx {
     double* sigw = nullptr;
     qk::Split3 Bsplit, BovTsplit, Tsplit;  // B (rows pq), Bov^T (rows P, k = jb), T (rows m)
     bool bsplit_valid = false;
-    // eigensolver: 0 = rocSOLVER dsyevd for every RPA (QuAcK's scheme); 1 = refine
+    // eigensolver: 0 = a full solve for every RPA (QuAcK's scheme); 1 = refine
     // the previous eigenvectors by Newton steps when the energies moved by at
-    // most eig_demax since they were computed, dsyevd otherwise or on failure
-    int eig_mode = 0;  // bit 0: refine; bit 1: own tridiagonalisation instead of dsyevd
+    // most eig_demax since they were computed, a full solve otherwise or on failure
+    int eig_mode = 0;  // bit 0: refine; bit 1: split-precision full solves by the own tridiagonalisation too
     double eig_demax = 5e-3;
-    double *Zev = nullptr, *tau = nullptr, *trd_work = nullptr, *orm_work = nullptr;  // own full-solve path
+    double* eigw = nullptr;  // work of the full solves, on first use
+    size_t eigw_doubles = 0;
+    double *Zev = nullptr, *tau = nullptr, *trd_work = nullptr, *orm_work = nullptr;  // split-precision full solves
     qk::SolveGraphs graphs;  // captured launch sequences of the own full solve
     double *Xv = nullptr, *Ym = nullptr, *Sm = nullptr, *Gm = nullptr, *lam = nullptr, *eig_dbuf = nullptr;
     int *perm = nullptr, *eig_ibuf = nullptr;

@@ -129,17 +129,15 @@ void gather_bov(hipStream_t s, const double* B, double* Bov, int naux, int n, in
 // Householder tridiagonalisation, upper triangle, LAPACK dsytrd layout (qk_sytrd.hip);
 // work holds sytrd_work_doubles(n, nb) doubles, nb <= 64.
 size_t sytrd_work_doubles(int n, int nb);
-// V (or null: none wanted): where ormtr_upper's work holds the reflectors.  With
-// resident, the last columns run in registers (qk_trdres.hip): no graph capture,
+// With resident, the last columns run in registers (qk_trdres.hip): no graph capture,
 // and one host wait.  Returns the order m of that part (0: none): its reflectors
-// are in V only, the others in A only.
+// are in V only (or nowhere, if null), the others in A only.
 int sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, double* V,
                 bool resident);
-// Z <- Q Z with the reflectors sytrd_upper left in A, TAU and, columns before m - 1,
-// in work (LAPACK dormtr, SIDE = 'L', UPLO = 'U', TRANS = 'N'); work holds
-// ormtr_work_doubles(n) and starts with V.
+// Z <- Q Z with the reflectors sytrd_upper (not resident) left in A, TAU (LAPACK
+// dormtr, SIDE = 'L', UPLO = 'U', TRANS = 'N'); work holds ormtr_work_doubles(n).
 size_t ormtr_work_doubles(int n);
-void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work, int m);
+void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work);
 // A symmetric from its upper triangle: A[i, j] = A[j, i] for i > j
 void sym_lower(hipStream_t s, double* A, int n);
 void permute_cols(hipStream_t s, const double* X, const int* perm, double* out, int n);
@@ -157,5 +155,36 @@ size_t trd_resident_words(int n, int batch);
 const int* trd_resident_fail(int n, int batch, const double* words);
 bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
                   long long sV, double* D, double* E, double* TAU, long long sd, int batch, double* words);
+
+// Eigenvalues (and eigenvectors) of batch symmetric tridiagonal matrices (qk_stedc.hip),
+// diagonals D and off-diagonals E sd apart, values ascending into w (may be D).
+// info[z] != 0: an entry of matrix z is not finite.  Z receives the eigenvectors
+// (n x n, sZ = n^2 apart), Z2 and U are scratch of the same shape.
+size_t tri_work_doubles(int n, int batch, bool vectors);
+void tri_values(hipStream_t s, int n, const double* D, const double* E, long long sd, int batch, double* w, long long sw,
+                double* work, int* info);
+void tri_vectors(hipStream_t s, int n, const double* D, const double* E, long long sd, int batch, double* w, long long sw,
+                 double* Z, double* Z2, long long sZ, double* U, long long sU, double* work, int* info);
+
+// Back-transformation with the columns of Z in registers (qk_ormstrip.hip), orders
+// up to orm_strip_max(): work of orm_strip_doubles(n) a matrix starts with V, leading
+// dimension orm_strip_ld(n); prepare takes reflectors j >= m - 1 from A, the others
+// (rows < m) are in V.
+int orm_strip_max();
+int orm_strip_ld(int n);
+size_t orm_strip_doubles(int n);
+void orm_strip_prepare(hipStream_t s, int n, int batch, const double* A, long long sA, const double* TAU, long long sT,
+                       double* work, int m);
+void orm_strip_apply(hipStream_t s, int n, int batch, double* Z, long long sZ, double* work);
+// Eigenvalues (ascending, w, sw apart) and, with vectors, eigenvectors (in A's place)
+// of batch symmetric matrices A (n x n, sA apart, upper triangle read, destroyed):
+// the own tridiagonalisation, divide and conquer or Sturm counts, and
+// back-transformation.  work: eigh_work_doubles(...); info[z] != 0: matrix z has an
+// entry that is not finite.  One host wait; not for graph capture.  tev (or null):
+// four events round the tridiagonalisation, the tridiagonal solve and the
+// back-transformation (the last two with vectors only).
+size_t eigh_work_doubles(int n, int batch, bool vectors);
+void eigh(hipStream_t s, int n, int batch, double* A, long long sA, double* w, long long sw, bool vectors, double* work,
+          int* info, hipEvent_t* tev = nullptr);
 
 }  // namespace qk

@@ -494,8 +494,13 @@ constexpr int OKC = 512;  // rows per split-K chunk of V^T Z
 
 // V (n x nbk, zero-padded columns past n-1) and the padded taus; rows < m of the
 // columns before m - 1 are in V already
-__global__ void k_build_v(const double* __restrict__ A, int n, const double* __restrict__ TAU, int nbk, int m,
-                          double* __restrict__ V, double* __restrict__ taup) {
+__global__ void k_build_v(const double* __restrict__ A, long long sA, int n, const double* __restrict__ TAU,
+                          long long sT, int nbk, int m, double* __restrict__ V, double* __restrict__ taup,
+                          long long sW) {
+    A += blockIdx.y * sA;
+    TAU += blockIdx.y * sT;
+    V += blockIdx.y * sW;
+    taup += blockIdx.y * sW;
     const long long total = (long long)n * nbk;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
          t += (long long)gridDim.x * blockDim.x) {
@@ -512,7 +517,10 @@ __global__ void k_build_v(const double* __restrict__ A, int n, const double* __r
 // Written OKS times side by side, [T T ... T] (OK x OKS OK), so that one GEMM
 // applies T to the sum of the split-K partials.
 __global__ __launch_bounds__(256) void k_build_t(const double* __restrict__ G, const double* __restrict__ taup,
-                                                 double* __restrict__ Trep, int oks) {
+                                                 double* __restrict__ Trep, int oks, long long sW) {
+    G += blockIdx.y * sW;
+    taup += blockIdx.y * sW;
+    Trep += blockIdx.y * sW;
     __shared__ double T[OK][OK + 1];
     __shared__ double gc[OK];
     const int b = blockIdx.x;
@@ -648,58 +656,171 @@ size_t ormtr_work_doubles(int n) {
            (size_t)OK * n;
 }
 
-void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work, int m) {
+namespace {
+// the parts of one matrix's back-transformation work
+struct OrmWork {
+    int nblk, nbk, oks;  // blocks of reflectors, padded reflectors, largest number of split-K chunks
+    double *V, *taup, *G, *Trep, *W1p, *W2;
+    OrmWork(int n, double* work) {
+        nblk = (n - 1 + OK - 1) / OK;
+        nbk = nblk * OK;
+        oks = (n + OKC - 1) / OKC;
+        V = work;
+        taup = V + (size_t)n * nbk;
+        G = taup + nbk;
+        Trep = G + (size_t)nblk * OK * OK;
+        W1p = Trep + (size_t)nblk * OK * OK * oks;  // (oks OK) x n, partial V^T Z stacked by chunk
+        W2 = W1p + (size_t)oks * OK * n;            // OK x n
+    }
+};
+}  // namespace
+
+void ormtr_prepare(hipStream_t s, int n, int batch, const double* A, long long sA, const double* TAU, long long sT,
+                   double* work, long long sW, int m) {
+    if (n == 1) return;
+    const OrmWork o(n, work);
+    const long long tot = (long long)n * o.nbk;
+    hipLaunchKernelGGL(k_build_v, dim3((unsigned)std::min<long long>((tot + 255) / 256, 65536), batch), dim3(256), 0, s, A,
+                       sA, n, TAU, sT, o.nbk, m, o.V, o.taup, sW);
+    QK_HIP(hipGetLastError());
+}
+
+void ormtr_apply(hipStream_t s, int n, int batch, double* Z, long long sZ, double* work, long long sW) {
     QK_CHECK(n >= 1, QK_E_ARG, "ormtr: bad size");
     if (n == 1) return;
-    const int nblk = (n - 1 + OK - 1) / OK;
-    const int nbk = nblk * OK;
-    const int oks = (n + OKC - 1) / OKC;  // largest number of split-K chunks
-    double* V = work;
-    double* taup = V + (size_t)n * nbk;
-    double* G = taup + nbk;
-    double* Trep = G + (size_t)nblk * OK * OK;
-    double* W1p = Trep + (size_t)nblk * OK * OK * oks;  // (oks OK) x n, partial V^T Z stacked by chunk
-    double* W2 = W1p + (size_t)oks * OK * n;            // OK x n
-    const long long tot = (long long)n * nbk;
-    hipLaunchKernelGGL(k_build_v, dim3((unsigned)std::min<long long>((tot + 255) / 256, 65536)), dim3(256), 0, s, A,
-                       n, TAU, nbk, m, V, taup);
-    QK_HIP(hipGetLastError());
+    const OrmWork o(n, work);
+    const int nblk = o.nblk, oks = o.oks;
     {
         Batch bg;
         bg.sa0 = (long long)OK * n;
         bg.sb0 = (long long)OK * n;
         bg.sc0 = (long long)OK * OK;
-        bg.count = nblk;
-        bg.zdiv = nblk;  // one-level batch: z0 = z runs over the sa0/sb0/sc0 strides
-        dgemm(s, true, false, OK, OK, n, 1.0, V, n, V, n, 0.0, G, OK, bg);
+        bg.sa1 = bg.sb1 = bg.sc1 = sW;
+        bg.count = nblk * batch;
+        bg.zdiv = nblk;  // z = block + nblk matrix
+        dgemm(s, true, false, OK, OK, n, 1.0, o.V, n, o.V, n, 0.0, o.G, OK, bg);
     }
-    hipLaunchKernelGGL(k_build_t, dim3(nblk), dim3(256), 0, s, G, taup, Trep, oks);
+    hipLaunchKernelGGL(k_build_t, dim3(nblk, batch), dim3(256), 0, s, o.G, o.taup, o.Trep, oks, sW);
     QK_HIP(hipGetLastError());
     const long long ldp = (long long)oks * OK;
     for (int b = 0; b < nblk; ++b) {
         const int j0 = b * OK;
         const int m = std::min(j0 + OK, n);
-        const double* Vb = V + (long long)n * j0;
+        const double* Vb = o.V + (long long)n * j0;
         // W1p = V(0:m, :)^T Z(0:m, :) in chunks of OKC rows, stacked
         const int s1 = m / OKC, rem = m % OKC;
+        Batch bz;  // one product per matrix
+        bz.count = batch;
         if (s1 > 0) {
             Batch bp;
             bp.sa0 = OKC;
             bp.sb0 = OKC;
             bp.sc0 = OK;
-            bp.count = s1;
+            bp.sa1 = sW;
+            bp.sb1 = sZ;
+            bp.sc1 = sW;
+            bp.count = s1 * batch;
             bp.zdiv = s1;
-            dgemm(s, true, false, OK, n, OKC, 1.0, Vb, n, Z, n, 0.0, W1p, ldp, bp);
+            dgemm(s, true, false, OK, n, OKC, 1.0, Vb, n, Z, n, 0.0, o.W1p, ldp, bp);
         }
-        if (rem > 0)
+        if (rem > 0) {
+            bz.sa1 = sW;
+            bz.sb1 = sZ;
+            bz.sc1 = sW;
             dgemm(s, true, false, OK, n, rem, 1.0, Vb + (long long)s1 * OKC, n, Z + (long long)s1 * OKC, n, 0.0,
-                  W1p + (long long)s1 * OK, ldp);
+                  o.W1p + (long long)s1 * OK, ldp, bz);
+        }
         const int sc = s1 + (rem > 0 ? 1 : 0);
         // W2 = T (sum of the partials) = [T ... T] W1p
-        dgemm(s, false, false, OK, n, sc * OK, 1.0, Trep + (long long)b * OK * OK * oks, OK, W1p, ldp, 0.0, W2, OK);
+        bz.sa1 = bz.sb1 = bz.sc1 = sW;
+        dgemm(s, false, false, OK, n, sc * OK, 1.0, o.Trep + (long long)b * OK * OK * oks, OK, o.W1p, ldp, 0.0, o.W2, OK,
+              bz);
         // Z(0:m, :) -= V(0:m, :) W2
-        dgemm(s, false, false, m, n, OK, -1.0, Vb, n, W2, OK, 1.0, Z, n);
+        bz.sc1 = sZ;
+        dgemm(s, false, false, m, n, OK, -1.0, Vb, n, o.W2, OK, 1.0, Z, n, bz);
     }
+}
+
+void ormtr_upper(hipStream_t s, int n, const double* A, const double* TAU, double* Z, double* work) {
+    ormtr_prepare(s, n, 1, A, 0, TAU, 0, work, 0, 0);
+    ormtr_apply(s, n, 1, Z, 0, work, 0);
+}
+
+// ---- full eigensolve ---------------------------------------------------------------------
+namespace {
+// work of eigh: the parts of all matrices, then the scratch of the launch-per-column form
+struct EighWork {
+    double *E, *TAU, *D, *tri, *words, *trd, *orm = nullptr, *Z2 = nullptr, *U = nullptr;
+    size_t total;
+    EighWork(int n, int batch, bool vectors, double* work) {
+        double* p = work;
+        const auto take = [&](size_t count) {
+            double* r = p;
+            p += (count + 1) & ~(size_t)1;
+            return r;
+        };
+        const size_t nb = (size_t)n * batch;
+        D = take(nb);
+        E = take(nb);
+        TAU = take(nb);
+        tri = take(tri_work_doubles(n, batch, vectors));
+        words = take(trd_resident_words(std::min(n, trd_resident_max()), batch));
+        trd = take(sytrd_work_doubles(n, 32));
+        if (vectors) {
+            orm = take((n <= orm_strip_max() ? orm_strip_doubles(n) : ormtr_work_doubles(n)) * batch);
+            Z2 = take(nb * n);
+            U = take(nb * n);
+        }
+        total = p - work;
+    }
+};
+}  // namespace
+
+size_t eigh_work_doubles(int n, int batch, bool vectors) { return EighWork(n, batch, vectors, nullptr).total; }
+
+void eigh(hipStream_t s, int n, int batch, double* A, long long sA, double* w, long long sw, bool vectors, double* work,
+          int* info, hipEvent_t* tev) {
+    QK_CHECK(n >= 1 && batch >= 1, QK_E_ARG, "eigh: bad size");
+    const EighWork k(n, batch, vectors, work);
+    // the columns of Z fit the registers up to order 2048; larger ones go through GEMMs
+    const bool strip = n <= orm_strip_max();
+    const int ldv = strip ? orm_strip_ld(n) : n;
+    const long long sW = strip ? orm_strip_doubles(n) : ormtr_work_doubles(n);
+    const auto prepare = [&](int z, int count, int m) {
+        if (!vectors) return;
+        double* wz = k.orm + z * sW;
+        const double *Az = A + z * sA, *tz = k.TAU + (long long)n * z;
+        if (strip) orm_strip_prepare(s, n, count, Az, sA, tz, n, wz, m);
+        else ormtr_prepare(s, n, count, Az, sA, tz, n, wz, sW, m);
+    };
+    if (tev) QK_HIP(hipEventRecord(tev[0], s));
+    int fail = 0;
+    const bool whole = trd_resident_fits(n);
+    if (whole && trd_resident(s, n, A, n, sA, k.orm, ldv, sW, k.D, k.E, k.TAU, n, batch, k.words)) {
+        QK_HIP(hipMemcpyAsync(&fail, trd_resident_fail(n, batch, k.words), sizeof(int), hipMemcpyDeviceToHost, s));
+        QK_HIP(hipStreamSynchronize(s));
+    }
+    if (whole && !fail) {
+        if (tev) QK_HIP(hipEventRecord(tev[1], s));
+        prepare(0, batch, n);
+    } else {
+        for (int z = 0; z < batch; ++z) {
+            const long long o = (long long)n * z;
+            const int m = sytrd_upper(s, n, A + z * sA, k.D + o, k.E + o, k.TAU + o, k.trd, 32,
+                                      vectors ? k.orm + z * sW : nullptr, !whole);
+            prepare(z, 1, m);
+        }
+        if (tev) QK_HIP(hipEventRecord(tev[1], s));
+    }
+    if (!vectors) {
+        tri_values(s, n, k.D, k.E, n, batch, w, sw, k.tri, info);
+        return;
+    }
+    tri_vectors(s, n, k.D, k.E, n, batch, w, sw, A, k.Z2, sA, k.U, (long long)n * n, k.tri, info);
+    if (tev) QK_HIP(hipEventRecord(tev[2], s));
+    if (strip) orm_strip_apply(s, n, batch, A, sA, k.orm);
+    else ormtr_apply(s, n, batch, A, sA, k.orm, sW);
+    if (tev) QK_HIP(hipEventRecord(tev[3], s));
 }
 
 }  // namespace qk

@@ -84,3 +84,27 @@ def test_full_solve_edges(nO, nV):
         tol2 = 0.5 * om_tolerance(ref2).sum() + nS * EPS * ref2["Om"].sum()
         assert abs(r["EcRPA"] - ref2["EcRPA"]) <= tol2, mode
     sys.stdout.flush()
+
+
+@pytest.mark.parametrize("coupling", [0.0, 1e-9, 1e-5, 1e-3])
+def test_full_solve_equal_poles(coupling):
+    """Evenly spaced orbital energies: most pair energies coincide, so that the divide and
+    conquer deflates nearly everything (coupling 0), rotates close poles, or
+    solves for roots next to their poles."""
+    from quack_amd import gw
+    print("full solve, equal poles, coupling", coupling, flush=True)
+    nO, nV = 9, 33
+    e, B = system(nO, nV, 3)
+    e = np.concatenate([-1.0 + 0.05 * np.arange(nO), 0.2 + 0.05 * np.arange(nV)])
+    B = B * (coupling / 0.02)
+    ref = reference(e, B, nO, True)
+    for mode in ("sytrd", "syevd"):
+        with gw.GWEngine(nO + nV, nO + nV, nO) as g:
+            g.set_eri_df(B)
+            g.set_eigensolver(mode)
+            g.screen(e)
+            sig, _ = g.sigma_at(e, e, eta=0.1)
+            r = g.g0w0(e, eta=0.1, linearize=True)
+        assert (np.abs(r["Om"] - ref["Om"]) <= om_tolerance(ref)).all(), mode
+        for s in (sig, r["SigC"]):
+            assert np.abs(s - ref["SigC"]).max() <= 1e-10 * np.abs(ref["SigC"]).max(), mode
