@@ -18,15 +18,23 @@ namespace qk {
 
 thread_local std::string g_last_error;
 
-// rocSOLVER dsyevd on the stream bound to rb; eigenvalues ascending in w.
-void syevd(hipStream_t s, rocblas_handle rb, bool vectors, int n, double* A, double* w, double* work, int* dinfo) {
-    rb_check(rocsolver_dsyevd(rb, vectors ? rocblas_evect_original : rocblas_evect_none, rocblas_fill_upper, n, A, n,
-                              w, work, dinfo),
-             "rocsolver_dsyevd");
+namespace {
+// rocSOLVER dsyevd with eigenvectors on the stream bound to rb; eigenvalues ascending in w.
+void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double* work, int* dinfo) {
+    rb_check(rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, n, A, n, w, work, dinfo), "rocsolver_dsyevd");
     int info = 0;
     QK_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
     QK_HIP(hipStreamSynchronize(s));
     QK_CHECK(info == 0, QK_E_EIG, "rocsolver_dsyevd failed, info = " + std::to_string(info));
+}
+}  // namespace
+
+void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, hipEvent_t* tev) {
+    eigh(s, n, 1, A, (long long)n * n, w, n, vectors, work, dinfo, tev);
+    int info = 0;
+    QK_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
+    QK_HIP(hipStreamSynchronize(s));
+    QK_CHECK(info == 0, QK_E_EIG, "eigensolver: the matrix has entries that are not finite");
 }
 
 // Tiny symmetric solve for DIIS: LU with partial pivoting; rcond is the exact
@@ -547,12 +555,7 @@ void solve_full(Ctx* c, bool vectors) {
         c->eigw = dalloc<double>(need);
         c->eigw_doubles = need;
     }
-    eigh(c->s, c->nS, 1, c->Cm, (long long)c->nS * c->nS, c->Om, c->nS, vectors, c->eigw, c->info,
-         c->eig_mode & 2 ? c->ev3 : nullptr);
-    int info = 0;
-    QK_HIP(hipMemcpyAsync(&info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->s));
-    QK_HIP(hipStreamSynchronize(c->s));
-    QK_CHECK(info == 0, QK_E_EIG, "eigensolver: the matrix has entries that are not finite");
+    eigh_checked(c->s, c->nS, c->Cm, c->Om, vectors, c->eigw, c->info, c->eig_mode & 2 ? c->ev3 : nullptr);
 }
 
 // The same for eigenvectors of a split-precision contraction, modes 2 and 3.
@@ -564,7 +567,7 @@ void solve_split(Ctx* c) {
         c->trd_work = dalloc<double>(sytrd_work_doubles(c->nS, 32));
         c->orm_work = dalloc<double>(ormtr_work_doubles(c->nS));
     }
-    syevd_own(c->s, c->rb, c->nS, c->Cm, c->Om, c->work, c->tau, c->Zev, c->trd_work, c->orm_work, c->info, c->ev3,
+    syevd_own(c->s, blas(c->rb, c->s), c->nS, c->Cm, c->Om, c->work, c->tau, c->Zev, c->trd_work, c->orm_work, c->info, c->ev3,
               &c->graphs);
 }
 
@@ -598,7 +601,7 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
             // makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
             const bool split = c->precision != 0 && vectors;
             if (split && !(c->eig_mode & 2)) {
-                syevd(c->s, c->rb, true, c->nS, c->Cm, c->Om, c->work, c->info);
+                syevd(c->s, blas(c->rb, c->s), c->nS, c->Cm, c->Om, c->work, c->info);
             } else {
                 if (split) solve_split(c);
                 else solve_full(c, vectors);
@@ -973,8 +976,6 @@ int qk_gw_create(qk_gw_handle* h, int nBas, int nOrb, int nC, int nO, int nV, in
         c->nBas = nBas; c->nOrb = nOrb; c->nC = nC; c->nO = nO; c->nV = nV; c->nR = nR; c->nS = nS;
         c->o = nO - nC; c->v = nOrb - nR - nO;
         QK_HIP(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking));
-        rb_check(rocblas_create_handle(&c->rb), "rocblas_create_handle");
-        rb_check(rocblas_set_stream(c->rb, c->s), "rocblas_set_stream");
         for (auto* e : {&c->ev[0], &c->ev[1], &c->ev2[0], &c->ev2[1], &c->ev3[0], &c->ev3[1], &c->ev3[2], &c->ev3[3]})
             QK_HIP(hipEventCreate(e));
         size_t n = nOrb, S = nS;
@@ -1472,7 +1473,6 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
     if (nS <= 0 || !Aph || (!TDA && !Bph) || !Om || !XpY || !XmY) return QK_E_ARG;
     return guarded(nullptr, [&] {
         hipStream_t s = scratch().s;
-        rocblas_handle rb = scratch().rb;
         size_t S2 = (size_t)nS * nS;
         std::vector<double*> bufs;
         auto get = [&](size_t cnt) { bufs.push_back(dalloc<double>(cnt)); return bufs.back(); };
@@ -1480,7 +1480,7 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
             double* A = get(S2);
             double* U = get(S2);
             double* w = get(nS);
-            double* work = get(nS);
+            double* work = get(eigh_work_doubles(nS, 1, true));
             double* sc = get(4);
             int* info = dalloc<int>(1);
             bufs.push_back(reinterpret_cast<double*>(info));
@@ -1489,7 +1489,7 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
             if (TDA) {
                 // LR/phRLR.f90:40-43
                 QK_HIP(hipMemcpyAsync(U, A, sizeof(double) * S2, hipMemcpyDeviceToDevice, s));
-                syevd(s, rb, true, nS, U, w, work, info);
+                eigh_checked(s, nS, U, w, true, work, info);
                 double* X = get(S2);
                 transpose(s, U, X, nS, nS, nS, nS);
                 rpa_finalize(s, w, nullptr, nullptr, sc, nS, 1, false);
@@ -1504,7 +1504,7 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
                 double* T = get(S2);
                 QK_HIP(hipMemcpyAsync(B, Bph, sizeof(double) * S2, hipMemcpyHostToDevice, s));
                 apb_amb(s, A, B, ApB, U, (long long)S2);
-                syevd(s, rb, true, nS, U, w, work, info);
+                eigh_checked(s, nS, U, w, true, work, info);
                 // LR/phRLR.f90:57-58: QuAcK warns when A - B has a negative
                 // eigenvalue and then takes its square root; stop before the
                 // NaN (or the infinite inverse root of a zero mode) spreads
@@ -1520,7 +1520,7 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
                 dgemm(s, false, true, nS, nS, nS, 1.0, T, nS, U, nS, 0.0, Iv, nS);   // ADAt(U, 1/sqrt(w))
                 dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, Sq, nS, 0.0, T, nS);  // tmp = ApB AmBSq
                 dgemm(s, false, false, nS, nS, nS, 1.0, Sq, nS, T, nS, 0.0, U, nS);    // Z = AmBSq tmp
-                syevd(s, rb, true, nS, U, w, work, info);
+                eigh_checked(s, nS, U, w, true, work, info);
                 rpa_finalize(s, w, nullptr, nullptr, sc, nS, 0, false);                 // Om = sqrt|w|
                 dgemm(s, true, false, nS, nS, nS, 1.0, U, nS, Sq, nS, 0.0, T, nS);     // XpY = Z^T AmBSq
                 rowscale_pow(s, T, w, nS, -0.5);

@@ -19,6 +19,8 @@ struct qk_gwb_ctx {
     double *K = nullptr, *dE = nullptr, *sd = nullptr, *Om0 = nullptr, *part = nullptr, *scal = nullptr;
     double* vec[10] = {};  // e, e0, eG, Sig, Z, eLin, eGW, w, f, df: nOrb per molecule
     int *info = nullptr, *active = nullptr, *nit = nullptr, *done = nullptr;
+    double* eigw = nullptr;  // work of the eigensolves, on first use
+    size_t eigw_doubles = 0;
     qk::Zs zs;
     int nchunk = 1;
     // evGW state on the device (qk_gwb_evgw): DIIS histories, per molecule
@@ -63,7 +65,7 @@ void release_batch(BCtx* b) {
     }
     b->mol.clear();
     for (double* p : {b->M, b->Cm, b->rhoT, b->Om, b->E, b->K, b->dE, b->sd, b->Om0, b->part, b->scal, b->hist, b->conv,
-                      b->outSig, b->outZ, b->outOm, b->outEc})
+                      b->outSig, b->outZ, b->outOm, b->outEc, b->eigw})
         if (p) (void)hipFree(p);
     for (double* p : b->vec)
         if (p) (void)hipFree(p);
@@ -73,22 +75,33 @@ void release_batch(BCtx* b) {
     if (b->s) (void)hipStreamDestroy(b->s);
 }
 
-// One strided-batched rocSOLVER dsyevd for every molecule; with check, the
-// info flags are read back (the graph-replayed evGW reads them after the cycle)
-void syevd_batched(BCtx* b, bool vectors, bool check) {
+// The eigensolves of every molecule together; with check, the info flags are
+// read back (the graph-replayed evGW reads them after the cycle).  Eigenvectors for
+// split-precision densities come from rocSOLVER's batched dsyevd, as a single
+// engine's keep their solver (screening, qk_gw_api.hip).
+void solve_batch(BCtx* b, bool vectors, bool check) {
     const int nS = b->mol[0]->nS;
     const long long S2 = (long long)nS * nS;
-    rb_check(rocsolver_dsyevd_strided_batched(b->rb, vectors ? rocblas_evect_original : rocblas_evect_none,
-                                              rocblas_fill_upper, nS, b->Cm, nS, S2, b->Om, nS, b->E, nS, b->info,
-                                              b->nmol),
-             "rocsolver_dsyevd_strided_batched");
+    if (b->precision != 0 && vectors) {
+        rb_check(rocsolver_dsyevd_strided_batched(blas(b->rb, b->s), rocblas_evect_original, rocblas_fill_upper, nS, b->Cm, nS, S2,
+                                                  b->Om, nS, b->E, nS, b->info, b->nmol),
+                 "rocsolver_dsyevd_strided_batched");
+    } else {
+        const size_t need = eigh_work_doubles(nS, b->nmol, vectors);
+        if (b->eigw_doubles < need) {
+            dfree(b->eigw);
+            b->eigw_doubles = 0;
+            b->eigw = dalloc<double>(need);
+            b->eigw_doubles = need;
+        }
+        eigh(b->s, nS, b->nmol, b->Cm, S2, b->Om, nS, vectors, b->eigw, b->info);
+    }
     if (check) {
         std::vector<int> info(b->nmol);
         QK_HIP(hipMemcpyAsync(info.data(), b->info, sizeof(int) * b->nmol, hipMemcpyDeviceToHost, b->s));
         QK_HIP(hipStreamSynchronize(b->s));
         for (int m = 0; m < b->nmol; ++m)
-            QK_CHECK(info[m] == 0, QK_E_EIG,
-                     "rocsolver_dsyevd_strided_batched failed for molecule " + std::to_string(m));
+            QK_CHECK(info[m] == 0, QK_E_EIG, "eigensolver failed for molecule " + std::to_string(m));
     }
 }
 
@@ -130,7 +143,7 @@ void screening_batch(BCtx* b, const double* e, int tda, bool vectors) {
     rpa_build_batch(b, e, tda);
     {
         BStage st(b, 1);
-        syevd_batched(b, vectors, true);
+        solve_batch(b, vectors, true);
     }
     rpa_finalize_batch(b, tda, vectors);
 }
@@ -241,8 +254,6 @@ int qk_gwb_create(qk_gwb_handle* h, int nmol, int nBas, int nOrb, int nC, int nO
         QK_CHECK(nmol <= 65535, QK_E_ARG, "at most 65535 molecules per batch");
         b->nmol = nmol;
         QK_HIP(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking));
-        rb_check(rocblas_create_handle(&b->rb), "rocblas_create_handle");
-        rb_check(rocblas_set_stream(b->rb, b->s), "rocblas_set_stream");
         const size_t n = nOrb, S = nS, nm = nmol;
         b->nchunk = sigma_chunks(nS, nOrb - nR - nC);
         b->zs.n = (long long)n;
@@ -273,7 +284,6 @@ int qk_gwb_create(qk_gwb_handle* h, int nmol, int nBas, int nOrb, int nC, int nO
             b->mol.push_back(c);
             c->shared = true;
             c->s = b->s;
-            c->rb = b->rb;
             c->nBas = nBas; c->nOrb = nOrb; c->nC = nC; c->nO = nO; c->nV = nV; c->nR = nR; c->nS = nS;
             c->o = nO - nC; c->v = nOrb - nR - nO;
             c->M = b->M + m * n * n * S;
@@ -484,7 +494,7 @@ int qk_gwb_evgw(qk_gwb_handle h, const double* eHF, const double* eGW_start, int
                 QK_HIP(hipGraphLaunch(h->gpre, s));
                 {
                     BStage se(h, 1);
-                    syevd_batched(h, true, false);
+                    solve_batch(h, true, false);
                 }
                 QK_HIP(hipGraphLaunch(h->gpost, s));
                 ++h->graph_cycles;
@@ -492,7 +502,7 @@ int qk_gwb_evgw(qk_gwb_handle h, const double* eHF, const double* eGW_start, int
                 pre();
                 {
                     BStage se(h, 1);
-                    syevd_batched(h, true, false);
+                    solve_batch(h, true, false);
                 }
                 post(false);
                 ++h->eager_cycles;
@@ -502,7 +512,7 @@ int qk_gwb_evgw(qk_gwb_handle h, const double* eHF, const double* eGW_start, int
             QK_HIP(hipStreamSynchronize(s));
             for (int m = 0; m < nm; ++m)
                 QK_CHECK(info[m] == 0, QK_E_EIG,
-                         "rocsolver_dsyevd_strided_batched failed for molecule " + std::to_string(m));
+                         "eigensolver failed for molecule " + std::to_string(m));
             bool any = false;
             for (int m = 0; m < nm; ++m) any = any || st[(size_t)m * 4] != 0;
             if (!any) break;

@@ -49,8 +49,18 @@ inline void rb_check(rocblas_status st, const char* what) {
     if (st != rocblas_status_success) throw Error{QK_E_HIP, std::string(what) + ": rocblas status " + std::to_string((int)st)};
 }
 
-// rocSOLVER dsyevd on the stream bound to rb; eigenvalues ascending in w.
-void syevd(hipStream_t s, rocblas_handle rb, bool vectors, int n, double* A, double* w, double* work, int* dinfo);
+// The handle in rb, bound to s; made on first use (split-precision full solves only).
+inline rocblas_handle blas(rocblas_handle& rb, hipStream_t s) {
+    if (!rb) {
+        rb_check(rocblas_create_handle(&rb), "rocblas_create_handle");
+        rb_check(rocblas_set_stream(rb, s), "rocblas_set_stream");
+    }
+    return rb;
+}
+
+// eigh of one n x n matrix, waited for; QK_E_EIG when it has entries that are not finite
+void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo,
+                  hipEvent_t* tev = nullptr);
 
 struct GraphSlot {
     const void* key = nullptr;
@@ -196,15 +206,10 @@ void upload_mo_block(hipStream_t s, const double* ERI_MO, double* M, int n, int 
 // rho(p,q,m) (QuAcK layout, host) into rhoT[m + nS (p + n q)] on the device (caller frees)
 double* upload_rho(hipStream_t s, const double* rho, int n, int nS);
 
-// Shared stream and rocBLAS handle of the handle-less entry points.
+// Shared stream of the handle-less entry points.
 struct Scratch {
     hipStream_t s = nullptr;
-    rocblas_handle rb = nullptr;
-    Scratch() {
-        QK_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-        rb_check(rocblas_create_handle(&rb), "rocblas_create_handle");
-        rb_check(rocblas_set_stream(rb, s), "rocblas_set_stream");
-    }
+    Scratch() { QK_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)); }
 };
 Scratch& scratch();
 

@@ -179,8 +179,6 @@ struct UScreen {
             c->v = n - nO[0];
             c->nS = nSt;
             QK_HIP(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking));
-            rb_check(rocblas_create_handle(&c->rb), "rocblas_create_handle");
-            rb_check(rocblas_set_stream(c->rb, c->s), "rocblas_set_stream");
             for (auto* e : {&c->ev[0], &c->ev[1], &c->ev2[0], &c->ev2[1], &c->ev3[0], &c->ev3[1], &c->ev3[2],
                             &c->ev3[3]})
                 QK_HIP(hipEventCreate(e));
