@@ -227,15 +227,21 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
                 a = b;
                 b = x;
             }
-            double c = 1.0, s = 0.0;
+            // Rutishauser's form (H. Rutishauser, Numer. Math. 9 (1966) 1): elements change by
+            // s times a correction, and the pivot's block by t a_pq, so that the small
+            // rotations of the last sweeps add next to no rounding
+            double s = 0.0, h = 0.0, na = 0.0, nb = 0.0;
             const bool on = pr < me / 2 && b < m;
             if (on) {
-                const double apq = A[a * LD + b];
+                const double apq = A[a * LD + b], app = A[a * LD + a], aqq = A[b * LD + b];
                 if (fabs(apq) > EPS * 0.125) {  // |T| is about 1
-                    const double th = (A[b * LD + b] - A[a * LD + a]) / (2.0 * apq);
+                    const double th = (aqq - app) / (2.0 * apq);
                     const double tt = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(1.0 + th * th));
-                    c = 1.0 / sqrt(1.0 + tt * tt);
+                    const double c = 1.0 / sqrt(1.0 + tt * tt);
                     s = tt * c;
+                    h = s / (1.0 + c);
+                    na = app - tt * apq;
+                    nb = aqq + tt * apq;
                     turned = true;
                 }
             }
@@ -243,19 +249,20 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
             if (s != 0.0)
                 for (int r = r0; r < m; r += 8) {
                     double x = A[r * LD + a], y = A[r * LD + b];
-                    A[r * LD + a] = c * x - s * y;
-                    A[r * LD + b] = s * x + c * y;
+                    A[r * LD + a] = x - s * (y + h * x);
+                    A[r * LD + b] = y + s * (x - h * y);
                     x = V[r * LD + a];
                     y = V[r * LD + b];
-                    V[r * LD + a] = c * x - s * y;
-                    V[r * LD + b] = s * x + c * y;
+                    V[r * LD + a] = x - s * (y + h * x);
+                    V[r * LD + b] = y + s * (x - h * y);
                 }
             __syncthreads();
             if (s != 0.0)
                 for (int r = r0; r < m; r += 8) {
                     const double x = A[a * LD + r], y = A[b * LD + r];
-                    A[a * LD + r] = c * x - s * y;
-                    A[b * LD + r] = s * x + c * y;
+                    const bool pa = r == a, pb = r == b;  // the pivot's own block
+                    A[a * LD + r] = pa ? na : pb ? 0.0 : x - s * (y + h * x);
+                    A[b * LD + r] = pb ? nb : pa ? 0.0 : y + s * (x - h * y);
                 }
             __syncthreads();
         }
