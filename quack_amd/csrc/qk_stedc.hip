@@ -52,6 +52,13 @@ __device__ inline double rcp2(double x) {
     return fma(r, fma(-x, r, 1.0), r);
 }
 
+// 1/sqrt(x) likewise
+__device__ inline double rsq2(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+
 // ---- scaling, bounds ----------------------------------------------------------
 // One block per matrix: a power-of-two scale that brings max |T| to [1/2, 1), the
 // Gershgorin interval, and info = 1 where an entry is not finite.
@@ -235,11 +242,11 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
             if (on) {
                 const double apq = A[a * LD + b], app = A[a * LD + a], aqq = A[b * LD + b];
                 if (fabs(apq) > EPS * 0.125) {  // |T| is about 1
-                    const double th = (aqq - app) / (2.0 * apq);
-                    const double tt = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(1.0 + th * th));
-                    const double c = 1.0 / sqrt(1.0 + tt * tt);
+                    const double th = (aqq - app) * rcp2(2.0 * apq), q = 1.0 + th * th;
+                    const double tt = copysign(rcp2(fabs(th) + q * rsq2(q)), th);
+                    const double c = rsq2(1.0 + tt * tt);
                     s = tt * c;
-                    h = s / (1.0 + c);
+                    h = s * rcp2(1.0 + c);
                     na = app - tt * apq;
                     nb = aqq + tt * apq;
                     turned = true;

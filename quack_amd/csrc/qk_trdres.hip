@@ -24,15 +24,17 @@
 // load).  Two buffers alternate: a workgroup can write column c-2 only after
 // it has read every workgroup's column c-1, which they publish after reading c.
 //
-// Two shapes of the same algorithm: k_trd_small (n <= 512) gives each wave its
-// own rows and all columns, so every sum over columns stays inside a wave and
-// a column costs one barrier; k_trd_wide (n <= 3072) spreads the columns over
-// the workgroup's 512 threads.
+// Two shapes of the same algorithm: k_trd_small (n <= 160) is one workgroup and
+// needs no exchange; k_trd_wide (n <= 3072) spreads the columns over the 512
+// threads of each of its workgroups.
 //
-// Bound: the exchange and the barriers of a column, not arithmetic or memory.
-// Measured per column: 1.4 us at n = 64, 2.5 at 160 (one workgroup), 3.3 at 225,
-// 3.6 at 324, 6.2 at 900, 6.8 at 1326, 7.5 at 2025, 8.1 at 3072; 24 matrices of 324
-// take 1.22 ms together, one 1.17.
+// Bound: the latency of a column's chain (two sums over the columns, three barriers, the
+// exchange), not arithmetic or memory.  What shortened it, at n = 900 from 5.6 to 3.0 ms:
+// row c-1 goes out before the reflector is worked out, and only y is polled for once the
+// row is there (5.1 -> 4.4 and 3.4 -> 2.9); 16 rows a workgroup instead of 32, no
+// branch between the rows of a group.
+// Measured per column: 1.3 us at n = 60, 2.0 at 128, 2.75 at 225, 2.9 at 324, 3.3 at 900,
+// 3.6 at 1326, 4.1 at 2025, 7.4 at 3072; 24 matrices of 324 take 1.28 ms, one 0.93.
 //
 // Waits end: a reader that sees no progress for SPIN_TICKS raises *fail, which
 // the other workgroups read, and all leave; the caller then runs sytrd_upper.
@@ -148,35 +150,43 @@ __device__ inline Reflector reflector(double alpha, double xx) {
         h.tau = 0.0;
         h.scale = 0.0;
     } else {
-        const double nrm = sqrt(alpha * alpha + xx);
+        // beta = -sign(alpha) |x|, tau = (beta - alpha) / beta, scale = 1 / (alpha - beta), from the
+        // hardware's reciprocal (square root) and Newton steps: every column waits for them
+        const double s = alpha * alpha + xx, a = fabs(alpha);
+        double r = __builtin_amdgcn_rsq(s);
+        r = fma(0.5 * r, fma(-s * r, r, 1.0), r);
+        r = fma(0.5 * r, fma(-s * r, r, 1.0), r);
+        double nrm = s * r;
+        nrm = fma(0.5 * r, fma(-nrm, nrm, s), nrm);
         h.beta = alpha >= 0.0 ? -nrm : nrm;
-        h.tau = (h.beta - alpha) / h.beta;
-        h.scale = 1.0 / (alpha - h.beta);
+        h.tau = fma(a, r, 1.0);
+        const double d = a + nrm;
+        double q = __builtin_amdgcn_rcp(d);
+        q = fma(q, fma(-d, q, 1.0), q);
+        q = fma(q, fma(-d, q, 1.0), q);
+        h.scale = alpha >= 0.0 ? q : -q;
     }
     return h;
 }
 
-// n <= 64 KC <= 512.  Wave q of workgroup g owns rows g + G (q + 8 j), j < R; lane l
-// holds columns l + 64 k of them.  Needs n <= 8 R G.
+// One workgroup per matrix: n <= 64 KC, n <= 8 R.  Wave q owns rows q + 8 j, j < R; lane l
+// holds columns l + 64 k of them.  Every wave has all columns, so all sums stay inside
+// a wave; y and row c-1 pass through LDS, one barrier a column.
 template <int KC, int R>
 __global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
-    static_assert(R % 4 == 0 && KC <= 8, "rows go in fours; one column a thread in the exchange");
+    static_assert(R % 4 == 0, "rows go in fours");
     __shared__ double ys[2][64 * KC], as[2][64 * KC];
-    __shared__ double vw[8][2][64 * KC];  // each wave's copy of v and w, for its rows' entries
-    __shared__ int quit;
-    const int G = p.G, z = blockIdx.x / G, g = blockIdx.x % G, n = p.n;
+    __shared__ double2 vw[8][64 * KC];  // each wave's copy of (v, w), for its rows' entries
+    const int z = blockIdx.x, n = p.n;
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
     const double* A = p.A + z * p.sA;
     double* V = p.V ? p.V + z * p.sV : nullptr;
     double *D = p.D + z * p.sd, *E = p.E + z * p.sd, *TAU = p.TAU + z * p.sd;
-    u64* X = p.X + (long long)z * 8 * n;
-    const bool writer = g == 0 && q == 0;
-    double* vq = vw[q][0];
-    double* wq = vw[q][1];
+    double2* vwq = vw[q];
     double a[R][KC], v[KC], vp[KC], wp[KC], x[KC];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int r = g + G * (q + 8 * j);
+        const int r = q + 8 * j;
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             const int col = lane + 64 * k;
@@ -184,101 +194,77 @@ __global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
         }
     }
     int c = n - 1;
-    double xx = 0.0, alpha = 0.0;
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
         const int col = lane + 64 * k;
         x[k] = col <= c ? A[col + p.lda * c] : 0.0;
         vp[k] = wp[k] = 0.0;
-        vq[col] = wq[col] = 0.0;
-        if (writer && col == c) D[c] = x[k];
+        vwq[col] = double2{0.0, 0.0};
+        if (q == 0 && col == c) D[c] = x[k];
     }
-    if (threadIdx.x == 0) quit = 0;
-    lds_barrier();
-    unsigned spins = 0;
     for (; c >= 1; --c) {
         const int par = c & 1;
+        if (q == ((c - 1) & 7)) {  // row c-1, brought up to date
+            const int jr = (c - 1) >> 3;
+            const double2 f = vwq[c - 1];
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+                if (j == jr)
+#pragma unroll
+                    for (int k = 0; k < KC; ++k) {
+                        const int col = lane + 64 * k;
+                        if (col < c) as[par][col] = a[j][k] - f.x * wp[k] - f.y * vp[k];
+                    }
+        }
         // reflector of column c from x
-        xx = 0.0;
-        double sel = 0.0;
+        double xx = 0.0, sel = 0.0;
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             const int col = lane + 64 * k;
             if (k == (c - 1) >> 6) sel = x[k];
             if (col < c - 1) xx += x[k] * x[k];
         }
-        alpha = lane_value(sel, (c - 1) & 63);
-        const Reflector h = reflector(alpha, wave_sum(xx));
+        const Reflector h = reflector(lane_value(sel, (c - 1) & 63), wave_sum(xx));
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             const int col = lane + 64 * k;
             v[k] = col < c - 1 ? x[k] * h.scale : (col == c - 1 ? 1.0 : 0.0);
         }
-        // update of the previous column and y = A v, row by row
+        // update of the previous column and y = A v, four rows at a time
 #pragma unroll
         for (int j0 = 0; j0 < R; j0 += 4) {
-            if (g + G * (q + 8 * j0) < c) {
+            if (q + 8 * j0 < c) {
                 double acc[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const int r = g + G * (q + 8 * (j0 + u));
+                    // (rows past c are done: their v and w are zero, and nobody takes their y)
+                    const double2 f = vwq[min(q + 8 * (j0 + u), n - 1)];
                     acc[u] = 0.0;
-                    if (r < c) {
-                        const double vr = vq[r], wr = wq[r];
 #pragma unroll
-                        for (int k = 0; k < KC; ++k) {
-                            const double t = a[j0 + u][k] - vr * wp[k] - wr * vp[k];
+                    for (int k = 0; k < KC; ++k)
+                        if (64 * k < c) {
+                            const double t = a[j0 + u][k] - f.x * wp[k] - f.y * vp[k];
                             a[j0 + u][k] = t;
                             acc[u] += t * v[k];
                         }
-                        if (r == c - 1) {  // this row goes to everyone
-#pragma unroll
-                            for (int k = 0; k < KC; ++k) {
-                                const int col = lane + 64 * k;
-                                if (col < c) {
-                                    if (G > 1) publish(X + 4LL * n * par + 2LL * n + 2 * col, a[j0 + u][k], c);
-                                    else as[par][col] = a[j0 + u][k];
-                                }
-                            }
-                        }
-                    }
                 }
                 const double y = wave_sum4(acc);
-                const int r = g + G * (q + 8 * (j0 + (lane >> 4)));
-                if ((lane & 15) == 0 && r < c) {
-                    if (G > 1) publish(X + 4LL * n * par + 2 * r, y, c);
-                    else ys[par][r] = y;
-                }
+                const int r = q + 8 * (j0 + (lane >> 4));
+                if ((lane & 15) == 0 && r < c) ys[par][r] = y;
             }
         }
-        if (V && g == c % G && q == ((c / G) & 7)) {
+        if (V && q == (c & 7)) {
 #pragma unroll
             for (int k = 0; k < KC; ++k) {
                 const int col = lane + 64 * k;
                 if (col < n) V[col + p.ldv * (c - 1)] = v[k];
             }
         }
-        if (writer && lane == 0) {
+        if (threadIdx.x == 0) {
             E[c - 1] = h.beta;
             TAU[c - 1] = h.tau;
         }
-        if (G > 1 && (int)threadIdx.x < c) {
-            const u64* w = X + 4LL * n * par + 2 * threadIdx.x;
-            double y = 0.0, ao = 0.0;
-            long long t0 = 0;
-            for (;;) {
-                const bool f1 = arrived(w, c, y), f2 = arrived(w + 2LL * n, c, ao);
-                if (f1 && f2) break;
-                if (give_up(spins, t0, p.fail)) {
-                    quit = 1;
-                    break;
-                }
-            }
-            ys[par][threadIdx.x] = y;
-            as[par][threadIdx.x] = ao;
-        }
         lds_barrier();
-        if (G > 1 && quit) return;
         // w = tau y - tau^2 (y . v) v / 2
         double y[KC], dot = 0.0;
         sel = 0.0;
@@ -301,9 +287,8 @@ __global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
         for (int k = 0; k < KC; ++k) {
             const int col = lane + 64 * k;
             x[k] = col < c ? x[k] - (v[k] * wl + wp[k]) : 0.0;  // v(c-1) = 1
-            if (writer && col == c - 1) D[c - 1] = x[k];
-            vq[col] = v[k];
-            wq[col] = wp[k];
+            if (q == 0 && col == c - 1) D[c - 1] = x[k];
+            vwq[col] = double2{v[k], wp[k]};
         }
     }
 }
@@ -313,7 +298,7 @@ __global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
 template <int KC, int R>
 __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
     static_assert(R % 4 == 0 && R <= 64, "rows go in fours");
-    __shared__ double vs[TT * KC], ws[TT * KC];
+    __shared__ double2 vw[TT * KC];  // (v, w)
     __shared__ double yp[8][R];
     __shared__ double red1[8], red2[8];
     __shared__ double ylast, xlast;
@@ -341,7 +326,7 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
         const int col = tid + TT * k;
         x[k] = col <= c ? A[col + p.lda * c] : 0.0;
         vp[k] = wp[k] = 0.0;
-        vs[col] = ws[col] = 0.0;
+        vw[col] = double2{0.0, 0.0};
         if (g == 0 && col == c) D[c] = x[k];
         if (col < c - 1) part += x[k] * x[k];
         if (col == c - 1) xlast = x[k];
@@ -353,6 +338,21 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
     unsigned spins = 0;
     for (; c >= 1; --c) {
         const int par = c & 1;
+        // row c-1, brought up to date, goes to everyone first: it is on its way while the
+        // reflector and y are worked out
+        if (g == (c - 1) % G) {
+            const int jr = (c - 1) / G;
+            const double2 f = vw[c - 1];
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+                if (j == jr)
+#pragma unroll
+                    for (int k = 0; k < KC; ++k) {
+                        const int col = tid + TT * k;
+                        const double t = a[j][k] - f.x * wp[k] - f.y * vp[k];
+                        if (col < c) publish(X + 4LL * n * par + 2LL * n + 2 * col, t, c);
+                    }
+        }
         double xx = 0.0;
 #pragma unroll
         for (int u = 0; u < 8; ++u) xx += red2[u];
@@ -368,25 +368,17 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
                 double acc[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const int r = g + G * (j0 + u);
+                    if (KC >= 5) __builtin_amdgcn_sched_barrier(0);  // registers for one row's loads at a time
+                    // (rows past c are done: their v and w are zero, and nobody takes their y)
+                    const double2 f = vw[min(g + G * (j0 + u), n - 1)];
                     acc[u] = 0.0;
-                    if (r < c) {
-                        const double vr = vs[r], wr = ws[r];
 #pragma unroll
-                        for (int k = 0; k < KC; ++k)
-                            if (TT * k < c) {
-                                const double t = a[j0 + u][k] - vr * wp[k] - wr * vp[k];
-                                a[j0 + u][k] = t;
-                                acc[u] += t * v[k];
-                            }
-                        if (r == c - 1) {
-#pragma unroll
-                            for (int k = 0; k < KC; ++k) {
-                                const int col = tid + TT * k;
-                                if (col < c) publish(X + 4LL * n * par + 2LL * n + 2 * col, a[j0 + u][k], c);
-                            }
+                    for (int k = 0; k < KC; ++k)
+                        if (TT * k < c) {
+                            const double t = a[j0 + u][k] - f.x * wp[k] - f.y * vp[k];
+                            a[j0 + u][k] = t;
+                            acc[u] += t * v[k];
                         }
-                    }
                 }
                 const double y = wave_sum4(acc);
                 if ((lane & 15) == 0) yp[q][j0 + (lane >> 4)] = y;
@@ -416,19 +408,24 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
         double y[KC], dot = 0.0;
         {
             long long t0 = 0;
+            const u64* w = X + 4LL * n * par + 2 * tid;
+            bool row = false;  // row c-1, sent early, is here
             for (;;) {
                 bool all = true;
+                if (!row) {
+                    row = true;
 #pragma unroll
-                for (int k = 0; k < KC; ++k) {
-                    const int col = tid + TT * k;
-                    y[k] = x[k] = 0.0;
-                    if (col < c) {
-                        const u64* w = X + 4LL * n * par + 2 * col;
-                        const bool f1 = arrived(w, c, y[k]), f2 = arrived(w + 2LL * n, c, x[k]);
-                        all = all && f1 && f2;
+                    for (int k = 0; k < KC; ++k) {
+                        x[k] = 0.0;
+                        if (tid + TT * k < c) row = arrived(w + 2LL * n + 2 * TT * k, c, x[k]) && row;
                     }
                 }
-                if (all) break;
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    y[k] = 0.0;
+                    if (tid + TT * k < c) all = arrived(w + 2 * TT * k, c, y[k]) && all;
+                }
+                if (all && row) break;
                 if (give_up(spins, t0, p.fail)) {
                     quit = 1;
                     break;
@@ -457,8 +454,7 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
             vp[k] = v[k];
             x[k] = col < c ? x[k] - (v[k] * wl + wp[k]) : 0.0;
             if (g == 0 && col == c - 1) D[c - 1] = x[k];
-            vs[col] = v[k];
-            ws[col] = wp[k];
+            vw[col] = double2{v[k], wp[k]};
             if (col < c - 2) part += x[k] * x[k];
             if (col == c - 2) xlast = x[k];
         }
@@ -498,32 +494,51 @@ void resident_gate(hipStream_t s, F&& launch) {
     QK_HIP(hipEventRecord(g.last[dev], s));
 }
 
+// Rows per workgroup and the kernel for them.  R KC register pairs hold a thread's share of
+// A (at most 80 of the 128 pairs; the rest are the column vectors).
+typedef void (*TrdKernel)(TrdArgs);
+struct Shape {
+    int top, rows;  // largest order, rows of a workgroup
+    TrdKernel k;
+};
+#define QK_SMALL(KC, R) {64 * KC, 8 * R, k_trd_small<KC, R>}
+#define QK_WIDE(KC, R) {TT * KC, R, k_trd_wide<KC, R>}
+// In each range of orders the fastest shape for one matrix first, then those that
+// take fewer workgroups a matrix: 12 matrices of order 474 take 2.0 ms with 16 rows (360
+// workgroups, two a CU) and 1.6 with 32, one takes 1.42 and 1.62.
+const Shape SHAPES[] = {
+    QK_SMALL(1, 8),  QK_SMALL(2, 16), {160, 160, k_trd_small<3, 20>},
+    QK_WIDE(1, 16),  QK_WIDE(1, 32),
+    QK_WIDE(2, 16),  QK_WIDE(2, 32),
+    QK_WIDE(3, 12),  QK_WIDE(3, 24),
+    QK_WIDE(4, 8),   QK_WIDE(4, 16),
+    QK_WIDE(5, 12),  QK_WIDE(6, 12)};
+
 int compute_units() {
     int dev = 0, cu = 0;
     QK_HIP(hipGetDevice(&dev));
     QK_HIP(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
     return cu;
 }
-
-// Workgroups per matrix.  R KC registers pairs hold a thread's share of A (at most 72
-// of the 128 pairs; the rest are the column vectors).  n <= 160 fits one
-// workgroup, which needs no exchange at all.
-struct Shape {
-    int kc, r, g;
-};
-Shape trd_shape(int n) {
-    if (n <= 64) return {1, 8, 1};
-    if (n <= 128) return {2, 16, 1};
-    if (n <= 160) return {3, 20, 1};
-    if (n <= 192) return {3, 12, 2};
-    if (n <= 256) return {4, 16, (n + 127) / 128};
-    if (n <= 384) return {6, 8, (n + 63) / 64};
-    if (n <= 512) return {8, 8, (n + 63) / 64};
-    if (n <= 1024) return {2, 32, (n + 31) / 32};
-    if (n <= 1536) return {3, 24, (n + 23) / 24};
-    if (n <= 2048) return {4, 16, (n + 15) / 16};
-    if (n <= 2560) return {5, 16, (n + 15) / 16};
-    return {6, 12, (n + 11) / 12};
+// workgroups of the kernel that the device holds at once
+int trd_capacity(TrdKernel k) {
+    int per = 0;
+    QK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k), TT, 0));
+    return per * compute_units();
+}
+// The first shape of n's range that gives every workgroup of the batch a CU of its own,
+// else its last one; null where one matrix does not fit the device.
+const Shape* trd_shape(int n, int batch) {
+    const int cu = compute_units();
+    const Shape* best = nullptr;
+    for (const Shape& s : SHAPES) {
+        if (n > s.top || (best && best->top != s.top)) continue;
+        const int g = (n + s.rows - 1) / s.rows;
+        if (g > cu) continue;
+        best = &s;
+        if (g == 1 || (long long)g * batch <= cu) break;
+    }
+    return best;
 }
 
 }  // namespace
@@ -533,16 +548,17 @@ size_t trd_resident_words(int n, int batch) { return 8 * (size_t)n * batch + 1; 
 const int* trd_resident_fail(int n, int batch, const double* words) {
     return reinterpret_cast<const int*>(words + trd_resident_words(n, batch) - 1);
 }
-bool trd_resident_fits(int n) { return n >= 1 && n <= trd_resident_max() && trd_shape(n).g <= compute_units(); }
+bool trd_resident_fits(int n) { return n >= 1 && n <= trd_resident_max() && trd_shape(n, 1) != nullptr; }
 
 bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
                   long long sV, double* D, double* E, double* TAU, long long sd, int batch, double* words) {
     QK_CHECK(trd_resident_fits(n) && lda >= n && (!V || ldv >= n) && batch >= 1, QK_E_ARG, "trd_resident: bad size");
-    const Shape sh = trd_shape(n);
+    const Shape& sh = *trd_shape(n, batch);
+    const int G = (n + sh.rows - 1) / sh.rows;
     u64* X = reinterpret_cast<u64*>(words);  // exchange words, then the flag of a wait given up
     int* fail = reinterpret_cast<int*>(words + trd_resident_words(n, batch) - 1);
-    const int per = sh.g > 1 ? std::max(1, compute_units() / sh.g) : batch;  // matrices of one launch
-    if (sh.g > 1) {
+    const int per = G > 1 ? std::max(1, trd_capacity(sh.k) / G) : batch;  // matrices of one launch
+    if (G > 1) {
         const long long cnt = (long long)trd_resident_words(n, batch);
         hipLaunchKernelGGL(k_zero_words, dim3((unsigned)std::min<long long>((cnt + 255) / 256, 1024)), dim3(256), 0, s, X,
                            cnt);
@@ -550,28 +566,15 @@ bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long lon
     }
     for (int b0 = 0; b0 < batch; b0 += per) {
         const int nb = std::min(per, batch - b0);
-        TrdArgs p{A + b0 * sA, lda, sA, n, sh.g, V ? V + b0 * sV : nullptr, ldv, sV, D + b0 * sd, E + b0 * sd,
+        TrdArgs p{A + b0 * sA, lda, sA, n, G, V ? V + b0 * sV : nullptr, ldv, sV, D + b0 * sd, E + b0 * sd,
                   TAU + b0 * sd, sd, X + 8LL * n * b0, fail};
-        const dim3 grid(sh.g * nb), blk(TT);
-        auto go = [&] {
-            if (n <= 64) hipLaunchKernelGGL((k_trd_small<1, 8>), grid, blk, 0, s, p);
-            else if (n <= 128) hipLaunchKernelGGL((k_trd_small<2, 16>), grid, blk, 0, s, p);
-            else if (n <= 160) hipLaunchKernelGGL((k_trd_small<3, 20>), grid, blk, 0, s, p);
-            else if (n <= 192) hipLaunchKernelGGL((k_trd_small<3, 12>), grid, blk, 0, s, p);
-            else if (n <= 256) hipLaunchKernelGGL((k_trd_small<4, 16>), grid, blk, 0, s, p);
-            else if (n <= 384) hipLaunchKernelGGL((k_trd_small<6, 8>), grid, blk, 0, s, p);
-            else if (n <= 512) hipLaunchKernelGGL((k_trd_small<8, 8>), grid, blk, 0, s, p);
-            else if (n <= 1024) hipLaunchKernelGGL((k_trd_wide<2, 32>), grid, blk, 0, s, p);
-            else if (n <= 1536) hipLaunchKernelGGL((k_trd_wide<3, 24>), grid, blk, 0, s, p);
-            else if (n <= 2048) hipLaunchKernelGGL((k_trd_wide<4, 16>), grid, blk, 0, s, p);
-            else if (n <= 2560) hipLaunchKernelGGL((k_trd_wide<5, 16>), grid, blk, 0, s, p);
-            else hipLaunchKernelGGL((k_trd_wide<6, 12>), grid, blk, 0, s, p);
-        };
-        if (sh.g > 1) resident_gate(s, go);
+        const dim3 grid(G * nb), blk(TT);
+        auto go = [&] { hipLaunchKernelGGL(sh.k, grid, blk, 0, s, p); };
+        if (G > 1) resident_gate(s, go);
         else go();
         QK_HIP(hipGetLastError());
     }
-    return sh.g > 1;
+    return G > 1;
 }
 
 }  // namespace qk

@@ -108,3 +108,26 @@ def test_full_solve_equal_poles(coupling):
         assert (np.abs(r["Om"] - ref["Om"]) <= om_tolerance(ref)).all(), mode
         for s in (sig, r["SigC"]):
             assert np.abs(s - ref["SigC"]).max() <= 1e-10 * np.abs(ref["SigC"]).max(), mode
+
+
+@pytest.mark.parametrize("nmol", [3, 40, 60])
+def test_batched_full_solve(nmol):
+    """nS = 171 a molecule: every workgroup a CU of its own (3), fewer workgroups a
+    matrix (40), more matrices than one launch holds (60)."""
+    from quack_amd import gw
+    print("batched full solve", nmol, flush=True)
+    nO, nV = 9, 19
+    n = nO + nV
+    sys_ = [system(nO, nV, 100 + m) for m in range(nmol)]
+    with gw.GWBatch(nmol, n, n, nO) as b:
+        for m, (_, B) in enumerate(sys_):
+            chem = np.einsum("Ppq,Prs->pqrs", B, B, optimize=True)
+            b.set_eri_mo(m, np.asfortranarray(chem.transpose(0, 2, 1, 3)))
+        r = b.g0w0(np.stack([e for e, _ in sys_]), eta=0.1, linearize=True)
+    for m, (e, B) in enumerate(sys_):
+        ref = reference(e, B, nO, True)
+        assert (np.abs(r["Om"][m] - ref["Om"]) <= om_tolerance(ref)).all(), m
+        assert np.abs(r["SigC"][m] - ref["SigC"]).max() <= 1e-10 * np.abs(ref["SigC"]).max(), m
+        ref2 = reference(r["eGW"][m], B, nO, False)
+        tol2 = 0.5 * om_tolerance(ref2).sum() + n * n * EPS * ref2["Om"].sum()
+        assert abs(r["EcRPA"][m] - ref2["EcRPA"]) <= tol2, m
