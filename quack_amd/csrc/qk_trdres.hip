@@ -1,7 +1,7 @@
 // Householder tridiagonalisation with the matrix held in registers (gfx950).
 //
 // Same result as sytrd_upper (qk_sytrd.hip; LAPACK dsytd2, UPLO = 'U'), for
-// matrices of order n <= TRD_MAX and for the leading TRD_MAX x TRD_MAX part
+// matrices of order n <= 3072 and for the leading block of that order
 // that is left of a larger one.  The launch-per-step form pays two launches
 // a column (about 16 us a column at n = 1326, whatever the work); here one
 // launch runs every column and the G workgroups that share a matrix meet once
@@ -26,20 +26,21 @@
 //
 // Two shapes of the same algorithm: k_trd_small (n <= 160) is one workgroup and
 // needs no exchange; k_trd_wide (n <= 3072) spreads the columns over the 512
-// threads of each of its workgroups.
+// or 256 threads of each of its workgroups.
 //
 // Bound: the latency of a column's chain (two sums over the columns, three barriers, the
 // exchange), not arithmetic or memory.  What shortened it, at n = 900 from 5.6 to 3.0 ms:
 // row c-1 goes out before the reflector is worked out, and only y is polled for once the
 // row is there (5.1 -> 4.4 and 3.4 -> 2.9); 16 rows a workgroup instead of 32, no
 // branch between the rows of a group.
-// Measured per column: 1.3 us at n = 60, 2.0 at 128, 2.75 at 225, 2.9 at 324, 3.3 at 900,
-// 3.6 at 1326, 4.1 at 2025, 7.4 at 3072; 24 matrices of 324 take 1.28 ms, one 0.93.
+// Measured per column: 1.1 us at n = 64, 1.6 at 128, 1.9 at 225, 2.3 at 324, 3.3 at 900,
+// 3.6 at 1326, 4.2 at 2025, 7.4 at 3072; 24 matrices of 324 take 1.05 ms, one 0.74.
+// About 45 % of a column is the wait for the others' y.
 //
 // Waits end: a reader that sees no progress for SPIN_TICKS raises *fail, which
 // the other workgroups read, and all leave; the caller then runs sytrd_upper.
 // Launches whose workgroups wait for each other are kept one after another on
-// the device (resident_gate), each with at most one workgroup per CU.
+// the device (resident_gate), each with no more workgroups than it holds.
 #include <mutex>
 
 #include "qk_kernels.h"
@@ -50,7 +51,7 @@ namespace {
 typedef unsigned long long u64;
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int TT = 512;  // threads per workgroup: two waves per SIMD, 256 VGPRs each
+constexpr int TT = 512;  // threads per CU: two waves per SIMD, 256 VGPRs each
 constexpr long long SPIN_TICKS = 200000000LL;  // 2 s of the 100 MHz clock
 
 __device__ inline void lds_barrier() {
@@ -99,6 +100,19 @@ __device__ inline double wave_sum4(const double* a) {
 __device__ inline double lane_value(double v, int lane) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// sum of N values st apart in LDS, N a power of two, as a tree
+template <int N>
+__device__ inline double tree_sum(const double* v, int st) {
+    double t[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) t[i] = v[i * st];
+#pragma unroll
+    for (int m = N / 2; m > 0; m /= 2)
+#pragma unroll
+        for (int i = 0; i < m; ++i) t[i] += t[i + m];
+    return t[0];
 }
 
 // one double with its column number beside either half
@@ -293,14 +307,14 @@ __global__ __launch_bounds__(TT) void k_trd_small(TrdArgs p) {
     }
 }
 
-// n <= 512 KC.  Workgroup g owns rows g + G j, j < R; thread t holds columns t + 512 k
+// n <= NT KC.  Workgroup g owns rows g + G j, j < R; thread t holds columns t + NT k
 // of them.  Needs n <= R G.
-template <int KC, int R>
-__global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
+template <int KC, int R, int NT>
+__global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
     static_assert(R % 4 == 0 && R <= 64, "rows go in fours");
-    __shared__ double2 vw[TT * KC];  // (v, w)
-    __shared__ double yp[8][R];
-    __shared__ double red1[8], red2[8];
+    __shared__ double2 vw[NT * KC];  // (v, w)
+    __shared__ double yp[NT / 64][R];
+    __shared__ double red1[NT / 64], red2[NT / 64];
     __shared__ double ylast, xlast;
     __shared__ int quit;
     const int G = p.G, z = blockIdx.x / G, g = blockIdx.x % G, n = p.n;
@@ -315,7 +329,7 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
         const int r = g + G * j;
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
-            const int col = tid + TT * k;
+            const int col = tid + NT * k;
             a[j][k] = r < n && col < n ? load_sym(A, p.lda, r, col) : 0.0;
         }
     }
@@ -323,7 +337,7 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
     double part = 0.0;
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
-        const int col = tid + TT * k;
+        const int col = tid + NT * k;
         x[k] = col <= c ? A[col + p.lda * c] : 0.0;
         vp[k] = wp[k] = 0.0;
         vw[col] = double2{0.0, 0.0};
@@ -348,18 +362,15 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
                 if (j == jr)
 #pragma unroll
                     for (int k = 0; k < KC; ++k) {
-                        const int col = tid + TT * k;
+                        const int col = tid + NT * k;
                         const double t = a[j][k] - f.x * wp[k] - f.y * vp[k];
                         if (col < c) publish(X + 4LL * n * par + 2LL * n + 2 * col, t, c);
                     }
         }
-        double xx = 0.0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) xx += red2[u];
-        const Reflector h = reflector(xlast, xx);
+        const Reflector h = reflector(xlast, tree_sum<NT / 64>(red2, 1));
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
-            const int col = tid + TT * k;
+            const int col = tid + NT * k;
             v[k] = col < c - 1 ? x[k] * h.scale : (col == c - 1 ? 1.0 : 0.0);
         }
 #pragma unroll
@@ -374,7 +385,7 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
                     acc[u] = 0.0;
 #pragma unroll
                     for (int k = 0; k < KC; ++k)
-                        if (TT * k < c) {
+                        if (NT * k < c) {
                             const double t = a[j0 + u][k] - f.x * wp[k] - f.y * vp[k];
                             a[j0 + u][k] = t;
                             acc[u] += t * v[k];
@@ -388,16 +399,13 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
         if (tid < R) {
             const int r = g + G * tid;
             if (r < c) {
-                double y = 0.0;
-#pragma unroll
-                for (int u = 0; u < 8; ++u) y += yp[u][tid];
-                publish(X + 4LL * n * par + 2 * r, y, c);
+                publish(X + 4LL * n * par + 2 * r, tree_sum<NT / 64>(&yp[0][tid], R), c);
             }
         }
         if (V && g == c % G) {
 #pragma unroll
             for (int k = 0; k < KC; ++k) {
-                const int col = tid + TT * k;
+                const int col = tid + NT * k;
                 if (col < n) V[col + p.ldv * (c - 1)] = v[k];
             }
         }
@@ -417,13 +425,13 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
 #pragma unroll
                     for (int k = 0; k < KC; ++k) {
                         x[k] = 0.0;
-                        if (tid + TT * k < c) row = arrived(w + 2LL * n + 2 * TT * k, c, x[k]) && row;
+                        if (tid + NT * k < c) row = arrived(w + 2LL * n + 2 * NT * k, c, x[k]) && row;
                     }
                 }
 #pragma unroll
                 for (int k = 0; k < KC; ++k) {
                     y[k] = 0.0;
-                    if (tid + TT * k < c) all = arrived(w + 2 * TT * k, c, y[k]) && all;
+                    if (tid + NT * k < c) all = arrived(w + 2 * NT * k, c, y[k]) && all;
                 }
                 if (all && row) break;
                 if (give_up(spins, t0, p.fail)) {
@@ -435,21 +443,19 @@ __global__ __launch_bounds__(TT) void k_trd_wide(TrdArgs p) {
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             dot += y[k] * v[k];
-            if (tid + TT * k == c - 1) ylast = y[k];
+            if (tid + NT * k == c - 1) ylast = y[k];
         }
         dot = wave_sum(dot);
         if (lane == 0) red1[q] = dot;
         lds_barrier();
         if (quit) return;
-        dot = 0.0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) dot += red1[u];
+        dot = tree_sum<NT / 64>(red1, 1);
         const double half = -0.5 * h.tau * h.tau * dot;
         const double wl = h.tau * ylast + half;  // w(c-1), v(c-1) = 1
         part = 0.0;
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
-            const int col = tid + TT * k;
+            const int col = tid + NT * k;
             wp[k] = h.tau * y[k] + half * v[k];
             vp[k] = v[k];
             x[k] = col < c ? x[k] - (v[k] * wl + wp[k]) : 0.0;
@@ -494,49 +500,49 @@ void resident_gate(hipStream_t s, F&& launch) {
     QK_HIP(hipEventRecord(g.last[dev], s));
 }
 
-// Rows per workgroup and the kernel for them.  R KC register pairs hold a thread's share of
-// A (at most 80 of the 128 pairs; the rest are the column vectors).
+// Rows and threads of a workgroup and the kernel for them.  R KC register pairs hold a
+// thread's share of A (at most 72 of the 128 pairs; the rest are the column vectors).
 typedef void (*TrdKernel)(TrdArgs);
 struct Shape {
-    int top, rows;  // largest order, rows of a workgroup
+    int top, rows, threads;  // largest order, rows and threads of a workgroup
     TrdKernel k;
 };
-#define QK_SMALL(KC, R) {64 * KC, 8 * R, k_trd_small<KC, R>}
-#define QK_WIDE(KC, R) {TT * KC, R, k_trd_wide<KC, R>}
-// In each range of orders the fastest shape for one matrix first, then those that
-// take fewer workgroups a matrix: 12 matrices of order 474 take 2.0 ms with 16 rows (360
-// workgroups, two a CU) and 1.6 with 32, one takes 1.42 and 1.62.
+#define QK_SMALL(KC, R) {64 * KC, 8 * R, TT, k_trd_small<KC, R>}
+#define QK_WIDE(KC, R, NT) {NT * KC, R, NT, k_trd_wide<KC, R, NT>}
+// In each range of orders the fastest shape for one matrix first, then those that take
+// fewer workgroups a matrix.  Four waves instead of eight, with twice the columns a thread,
+// halve the sums over a row and the barriers' skew (n = 225: 0.56 -> 0.50 ms, with 8
+// rows 0.43; n = 474: 1.23 -> 1.17), up to where a thread's longer rows cost
+// more (n = 1326: 4.8 -> 5.7).
 const Shape SHAPES[] = {
-    QK_SMALL(1, 8),  QK_SMALL(2, 16), {160, 160, k_trd_small<3, 20>},
-    QK_WIDE(1, 16),  QK_WIDE(1, 32),
-    QK_WIDE(2, 16),  QK_WIDE(2, 32),
-    QK_WIDE(3, 12),  QK_WIDE(3, 24),
-    QK_WIDE(4, 8),   QK_WIDE(4, 16),
-    QK_WIDE(5, 12),  QK_WIDE(6, 12)};
+    QK_SMALL(1, 8),      QK_SMALL(2, 16),     {160, 160, TT, k_trd_small<3, 20>},
+    QK_WIDE(1, 8, 256),  QK_WIDE(1, 16, 256), QK_WIDE(1, 32, 256),
+    QK_WIDE(2, 8, 256),  QK_WIDE(2, 16, 256), QK_WIDE(2, 32, 256),
+    {1024, 8, 256, k_trd_wide<4, 8, 256>},    QK_WIDE(2, 16, 512), QK_WIDE(2, 32, 512),
+    QK_WIDE(3, 12, 512), QK_WIDE(3, 24, 512),
+    QK_WIDE(4, 8, 512),  QK_WIDE(4, 16, 512),
+    QK_WIDE(5, 12, 512), QK_WIDE(6, 12, 512)};
 
-int compute_units() {
+// Matrices whose workgroups a launch holds at once: one of 512 or two of 256 threads a CU
+// (what 256 registers a lane allow).
+int trd_at_once(const Shape& s, int g) {
     int dev = 0, cu = 0;
     QK_HIP(hipGetDevice(&dev));
     QK_HIP(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
-    return cu;
+    return cu * (TT / s.threads) / g;
 }
-// workgroups of the kernel that the device holds at once
-int trd_capacity(TrdKernel k) {
-    int per = 0;
-    QK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k), TT, 0));
-    return per * compute_units();
-}
-// The first shape of n's range that gives every workgroup of the batch a CU of its own,
-// else its last one; null where one matrix does not fit the device.
+// The first shape of n's range that takes the whole batch at once, else its last one:
+// 24 matrices of order 324 take 1.53 ms with 8 rows a workgroup (four a CU), 1.05
+// with 16, 1.22 with 32; 12 of order 474 2.13, 1.55 and 1.68.  Null where one
+// matrix does not fit the device.
 const Shape* trd_shape(int n, int batch) {
-    const int cu = compute_units();
     const Shape* best = nullptr;
     for (const Shape& s : SHAPES) {
         if (n > s.top || (best && best->top != s.top)) continue;
-        const int g = (n + s.rows - 1) / s.rows;
-        if (g > cu) continue;
+        const int g = (n + s.rows - 1) / s.rows, most = trd_at_once(s, g);
+        if (g > 1 && most < 1) continue;
         best = &s;
-        if (g == 1 || (long long)g * batch <= cu) break;
+        if (g == 1 || batch <= most) break;
     }
     return best;
 }
@@ -557,7 +563,7 @@ bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long lon
     const int G = (n + sh.rows - 1) / sh.rows;
     u64* X = reinterpret_cast<u64*>(words);  // exchange words, then the flag of a wait given up
     int* fail = reinterpret_cast<int*>(words + trd_resident_words(n, batch) - 1);
-    const int per = G > 1 ? std::max(1, trd_capacity(sh.k) / G) : batch;  // matrices of one launch
+    const int per = G > 1 ? std::min(batch, trd_at_once(sh, G)) : batch;  // matrices of one launch
     if (G > 1) {
         const long long cnt = (long long)trd_resident_words(n, batch);
         hipLaunchKernelGGL(k_zero_words, dim3((unsigned)std::min<long long>((cnt + 255) / 256, 1024)), dim3(256), 0, s, X,
@@ -568,7 +574,7 @@ bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long lon
         const int nb = std::min(per, batch - b0);
         TrdArgs p{A + b0 * sA, lda, sA, n, G, V ? V + b0 * sV : nullptr, ldv, sV, D + b0 * sd, E + b0 * sd,
                   TAU + b0 * sd, sd, X + 8LL * n * b0, fail};
-        const dim3 grid(G * nb), blk(TT);
+        const dim3 grid(G * nb), blk(sh.threads);
         auto go = [&] { hipLaunchKernelGGL(sh.k, grid, blk, 0, s, p); };
         if (G > 1) resident_gate(s, go);
         else go();
