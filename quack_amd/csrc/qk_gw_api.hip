@@ -734,7 +734,8 @@ void qp_graph(Ctx* c, const double* e0, const double* eG, const double* start, d
     // the host reads the active count after every QP_SYNC_EVERY sweeps: the
     // sweeps issued after the last orbital finished are masked no-ops, so the
     // results are those of a read after every sweep
-    int h_active = 1;
+    int h_active = !qp_newton(c->s, c->rhoT, c->rho_f32, e0, eG, c->Om, eta, srg, flow, n, c->nC, c->nO, c->nR, c->nS, c->w,
+                              c->f, c->df, c->nit, c->done, QP_THRESH, QP_MAXIT);
     for (int it = 0; it < QP_MAXIT && h_active > 0;) {
         for (int k = 0; k < QP_SYNC_EVERY && it < QP_MAXIT; ++k, ++it) {
             sigma_partial(c->s, c->rhoT, c->rho_f32, c->w, eG, c->Om, c->done, eta, srg, flow, n, c->nC, c->nO, c->nR,

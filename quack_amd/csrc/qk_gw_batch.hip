@@ -202,8 +202,11 @@ void qp_graph_batch(BCtx* b, double eta, int srg, const double* eG, const double
     Ctx* c0 = b->mol[0];
     const int nm = b->nmol, n = c0->nOrb;
     qp_init(b->s, start, b->vec[V_W], b->vec[V_F], b->nit, b->done, n, c0->nC, c0->nR, b->zs, nm);
+    const bool one = qp_newton(b->s, b->rhoT, b->precision != 0, b->vec[V_E0], eG, b->Om, eta, srg, SRG_FLOW, n, c0->nC,
+                               c0->nO, c0->nR, c0->nS, b->vec[V_W], b->vec[V_F], b->vec[V_DF], b->nit, b->done, QP_THRESH,
+                               QP_MAXIT, b->zs, nm);
     std::vector<int> act(nm, 1);
-    for (int it = 0; it < QP_MAXIT; ++it) {
+    for (int it = 0; it < QP_MAXIT && !one; ++it) {
         sigma_partial(b->s, b->rhoT, b->precision != 0, b->vec[V_W], eG, b->Om, b->done, eta, srg, SRG_FLOW, n, c0->nC,
                       c0->nO, c0->nR, c0->nS, b->nchunk, b->part, b->zs, nm);
         qp_update(b->s, b->part, b->nchunk, b->vec[V_E0], b->vec[V_W], b->vec[V_F], b->vec[V_DF], b->nit, b->done, n,

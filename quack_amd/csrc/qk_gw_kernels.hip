@@ -406,6 +406,96 @@ __global__ void k_qp_update(const double* __restrict__ part, int nchunk, const d
     if (threadIdx.x == 0) active[0] = (int)r;
 }
 
+// All Newton steps of an orbital in one workgroup: the sweep over its rho(p, :, :), the
+// step and the stop are GW/RGW_QP_graph.f90:50-92 as k_sigma_partial and k_qp_update have
+// them, a launch pair a step and a host read every few, which took 60 us a step for 24
+// molecules of 60 orbitals and 324 modes (64 steps where an SRG solve fails: 4 ms) where
+// the arithmetic of a step is about 3.  Sixteen waves share the rows q, a wave takes
+// four modes a lane at a time.  Bound: a row's load latency (rho stays in the caches).
+constexpr int QPN = 1024;
+__global__ __launch_bounds__(QPN) void k_qp_newton(const double* __restrict__ rhoT, const double* __restrict__ eHF,
+                                                   const double* __restrict__ e, const double* __restrict__ Om, double eta,
+                                                   int srg, double flow, int n, int nC, int nO, int nR, int nS,
+                                                   double* __restrict__ w, double* __restrict__ f,
+                                                   double* __restrict__ df, int* __restrict__ nit, int* __restrict__ done,
+                                                   double thresh, int maxit, Zs zs) {
+    __shared__ double sh[2][2 * QPN / 64];
+    {
+        const long long z = blockIdx.z;
+        rhoT += z * zs.R;
+        eHF += z * zs.n;
+        e += z * zs.n;
+        Om += z * zs.S;
+        w += z * zs.n;
+        f += z * zs.n;
+        df += z * zs.n;
+        nit += z * zs.n;
+        done += z * zs.n;
+    }
+    const int p = nC + blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const double eta2 = eta * eta, e0 = eHF[p];
+    double wp = w[p], fp = 1.0, dfp = 0.0;
+    int it = 0;
+    do {
+        double s = 0.0, d = 0.0;
+        for (int q = nC + wv; q < n - nR; q += QPN / 64) {
+            const double* row = rhoT + (long long)nS * (p + (long long)n * q);
+            const double sgn = q < nO ? 1.0 : -1.0, wq = wp - e[q];
+            for (int m0 = lane; m0 - lane < nS; m0 += 256) {
+                double r[4], om[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {  // (past the end: the last mode, unused)
+                    const int m = min(m0 + 64 * k, nS - 1);
+                    r[k] = row[m];
+                    om[k] = Om[m];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (m0 + 64 * k >= nS) continue;
+                    const double num = 2.0 * r[k] * r[k], eps = wq + sgn * om[k], e2 = eps * eps;
+                    if (!srg) {
+                        const double den = recip(e2 + eta2);
+                        s += num * eps * den;
+                        d -= num * (e2 - eta2) * den * den;
+                    } else {
+                        const double x = 2.0 * flow * e2;
+                        const double g = x > 38.0 ? 1.0 : 1.0 - exp(-x);
+                        const double inv = recip(eps), reg = num * g * inv;
+                        s += reg;
+                        d -= reg * inv;
+                    }
+                }
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            s += __shfl_xor(s, o, 64);
+            d += __shfl_xor(d, o, 64);
+        }
+        double* b = sh[it & 1];  // the other half may still be read
+        if (lane == 0) {
+            b[2 * wv] = s;
+            b[2 * wv + 1] = d;
+        }
+        __syncthreads();
+        s = d = 0.0;
+        for (int k = 0; k < QPN / 64; ++k) {
+            s += b[2 * k];
+            d += b[2 * k + 1];
+        }
+        ++it;
+        fp = wp - e0 - s;
+        dfp = 1.0 / (1.0 - d);
+        wp -= dfp * fp;
+    } while (fabs(fp) > thresh && it < maxit);  // the same in every thread
+    if (threadIdx.x == 0) {
+        w[p] = wp;
+        f[p] = fp;
+        df[p] = dfp;
+        nit[p] = it;
+        done[p] = 1;
+    }
+}
+
 // eGW(p) = w, Z(p) = df unless nIt == maxIt (then eGW = eGWlin, Z kept)
 __global__ void k_qp_finish(const double* __restrict__ w, const double* __restrict__ df, const int* __restrict__ nit,
                             const double* __restrict__ eGWlin, const double* __restrict__ eG,
@@ -1121,6 +1211,19 @@ void qp_init(hipStream_t s, const double* eGWlin, double* w, double* f, int* nit
     hipLaunchKernelGGL(k_qp_init, dim3((n + 255) / 256, 1, nz), dim3(256), 0, s, eGWlin, w, f, nit, done, n, nC, nR,
                        zs);
     QK_HIP(hipGetLastError());
+}
+bool qp_newton(hipStream_t s, const void* rhoT, bool rho_f32, const double* eHF, const double* eG, const double* Om,
+               double eta, int srg, double flow, int n, int nC, int nO, int nR, int nS, double* w, double* f, double* df,
+               int* nit, int* done, double thresh, int maxit, const Zs& zs, int nz) {
+    // One CU reads an orbital's rho at some 50 GB/s: above 4 MB an orbital the chunked sweeps,
+    // which spread an orbital over the chip, are faster once few orbitals are left.  FP32
+    // densities keep them too: their callers' results depend on every bit.
+    const int nact = n - nR - nC;
+    if (rho_f32 || (long long)nact * nS > (1 << 19)) return false;
+    hipLaunchKernelGGL(k_qp_newton, dim3(nact, 1, nz), dim3(QPN), 0, s, static_cast<const double*>(rhoT), eHF, eG, Om, eta,
+                       srg, flow, n, nC, nO, nR, nS, w, f, df, nit, done, thresh, maxit, zs);
+    QK_HIP(hipGetLastError());
+    return true;
 }
 void qp_update(hipStream_t s, const double* part, int nchunk, const double* eHF, double* w, double* f, double* df,
                int* nit, int* done, int n, double thresh, int maxit, int* active, const Zs& zs, int nz) {

@@ -68,7 +68,8 @@ void qp_dev(hipStream_t s, QpWork& q, const double* rT, const double* dO, int do
     QK_HIP(hipMemcpyAsync(q.eL, eGWlin, sizeof(double) * n, hipMemcpyHostToDevice, s));
     QK_HIP(hipMemcpyAsync(q.z, Z, sizeof(double) * n, hipMemcpyHostToDevice, s));
     qp_init(s, q.eL, q.w, q.f, q.nit, q.done, n, nC, nR);
-    int h_active = 1;
+    int h_active = !qp_newton(s, rT, false, q.e0, q.eG, dO, eta, doSRG, flow, n, nC, nO, nR, nS, q.w, q.f, q.df, q.nit,
+                              q.done, QP_THRESH, QP_MAXIT);
     for (int it = 0; it < QP_MAXIT && h_active > 0;) {
         for (int k = 0; k < QP_SYNC_EVERY && it < QP_MAXIT; ++k, ++it) {
             sigma_partial(s, rT, false, q.w, q.eG, dO, q.done, eta, doSRG, flow, n, nC, nO, nR, nS, q.nch, q.part);

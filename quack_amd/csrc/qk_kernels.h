@@ -81,6 +81,11 @@ void bse_dyn(hipStream_t s, const double* rhoT, const double* OmR, const double*
              const double* Y, double Om, double eta, int n, int nO, int nS, int dtda, double* part);
 void qp_init(hipStream_t s, const double* eGWlin, double* w, double* f, int* nit, int* done, int n, int nC, int nR,
              const Zs& zs = Zs(), int nz = 1);
+// Every Newton step of every active orbital after qp_init, in one launch; false (nothing
+// launched) where the sweeps of sigma_partial and qp_update are the better or the only form
+bool qp_newton(hipStream_t s, const void* rhoT, bool rho_f32, const double* eHF, const double* eG, const double* Om,
+               double eta, int srg, double flow, int n, int nC, int nO, int nR, int nS, double* w, double* f, double* df,
+               int* nit, int* done, double thresh, int maxit, const Zs& zs = Zs(), int nz = 1);
 void qp_update(hipStream_t s, const double* part, int nchunk, const double* eHF, double* w, double* f, double* df,
                int* nit, int* done, int n, double thresh, int maxit, int* active, const Zs& zs = Zs(), int nz = 1);
 // eG: energies in G; frozen orbitals of eGW are set to them (eOld in evGW).

@@ -2,10 +2,10 @@
 // iteration of GW/RGW_QP_graph.f90:50-92 on device-resident inputs, for
 // callers that cannot allocate device memory (code under hipGraph capture,
 // serving loops, harnesses that forbid hipMalloc).  It runs the same kernels
-// as qk_rgw_qp_graph (k_sigma_partial, k_qp_update, k_qp_init, k_qp_finish)
-// with their Newton state and partial sums in a library-owned static device
-// array, and a fixed QP_MAXIT = 64 sweeps whose finished orbitals are masked
-// on the device (the kernels skip them), so no host synchronisation or
+// as qk_rgw_qp_graph (qp_init, then k_qp_newton or k_sigma_partial and
+// k_qp_update, qp_finish) with their Newton state and partial sums in a
+// library-owned static device array, and in the sweeps' form a fixed QP_MAXIT = 64
+// of them whose finished orbitals are masked on the device, so no host synchronisation or
 // allocation happens inside: the call only enqueues work on the caller's
 // stream.  Every call on one GPU shares that GPU's array; calls that overlap
 // on one GPU race.
@@ -83,7 +83,9 @@ int qk_rgw_qp_graph_noalloc(int doSRG, double eta, double flow, int nOrb, int nC
         // qp_init writes w, f, nit and done before any read: nothing in the
         // shared array has to start at zero, whatever the last call left
         qp_init(s, eGWlin, w, f, nit, done, nOrb, nC, nR);
-        for (int it = 0; it < QP_MAXIT; ++it) {
+        const bool one = qp_newton(s, rhoT, false, eHF, eOld, Om, eta, doSRG, flow, nOrb, nC, nO, nR, nS, w, f, df, nit, done,
+                                   QP_THRESH, QP_MAXIT);
+        for (int it = 0; it < QP_MAXIT && !one; ++it) {
             sigma_partial(s, rhoT, false, w, eOld, Om, done, eta, doSRG, flow, nOrb, nC, nO, nR, nS, nchunk, part);
             qp_update(s, part, nchunk, eHF, w, f, df, nit, done, nOrb, QP_THRESH, QP_MAXIT, active);
         }
