@@ -18,8 +18,6 @@ namespace qk {
 
 thread_local std::string g_last_error;
 
-namespace {
-// rocSOLVER dsyevd with eigenvectors on the stream bound to rb; eigenvalues ascending in w.
 void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double* work, int* dinfo) {
     rb_check(rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, n, A, n, w, work, dinfo), "rocsolver_dsyevd");
     int info = 0;
@@ -27,7 +25,6 @@ void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double
     QK_HIP(hipStreamSynchronize(s));
     QK_CHECK(info == 0, QK_E_EIG, "rocsolver_dsyevd failed, info = " + std::to_string(info));
 }
-}  // namespace
 
 void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, hipEvent_t* tev) {
     eigh(s, n, 1, A, (long long)n * n, w, n, vectors, work, dinfo, tev);
@@ -599,7 +596,11 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
             // had: the slices round by the vectors' last bits and signs, which differ from
             // solver to solver (2e-11 of a self-energy on the H50 lattice), and evGW's DIIS
             // makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
-            const bool split = c->precision != 0 && vectors;
+            // qsGW keeps it too: its cycle can amplify the last bits of the vectors without
+            // bound where it does not converge (of 24 starts of a compressed H4 chain that
+            // differ by 1e-14, 8 converge within 64 cycles and 16 end anywhere), so its
+            // course from a given start stays the one it has always had.
+            const bool split = (c->precision != 0 || c->keep_syevd) && vectors;
             if (split && !(c->eig_mode & 2)) {
                 syevd(c->s, blas(c->rb, c->s), c->nS, c->Cm, c->Om, c->work, c->info);
             } else {

@@ -49,7 +49,7 @@ inline void rb_check(rocblas_status st, const char* what) {
     if (st != rocblas_status_success) throw Error{QK_E_HIP, std::string(what) + ": rocblas status " + std::to_string((int)st)};
 }
 
-// The handle in rb, bound to s; made on first use (split-precision full solves only).
+// The handle in rb, bound to s; made on first use (dsyevd: split-precision full solves and qsGW only).
 inline rocblas_handle blas(rocblas_handle& rb, hipStream_t s) {
     if (!rb) {
         rb_check(rocblas_create_handle(&rb), "rocblas_create_handle");
@@ -58,6 +58,8 @@ inline rocblas_handle blas(rocblas_handle& rb, hipStream_t s) {
     return rb;
 }
 
+// rocSOLVER dsyevd with eigenvectors on the stream bound to rb; eigenvalues ascending in w
+void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double* work, int* dinfo);
 // eigh of one n x n matrix, waited for; QK_E_EIG when it has entries that are not finite
 void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo,
                   hipEvent_t* tev = nullptr);
@@ -151,7 +153,8 @@ struct qk_gw_ctx {
     // most eig_demax since they were computed, a full solve otherwise or on failure
     int eig_mode = 0;  // bit 0: refine; bit 1: split-precision full solves by the own tridiagonalisation too
     double eig_demax = 5e-3;
-    double* eigw = nullptr;  // work of the full solves, on first use
+    bool keep_syevd = false;  // qsGW's engine: eigenvectors from rocSOLVER dsyevd
+    double* eigw = nullptr;   // work of the full solves, on first use
     size_t eigw_doubles = 0;
     double *Zev = nullptr, *tau = nullptr, *trd_work = nullptr, *orm_work = nullptr;  // split-precision full solves
     qk::SolveGraphs graphs;  // captured launch sequences of the own full solve

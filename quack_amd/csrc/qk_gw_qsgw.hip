@@ -15,9 +15,10 @@ struct qk_qsgw_ctx {
     qk_gw_handle g = nullptr;
     qk_scf_handle jk = nullptr;
     hipStream_t s = nullptr;
+    rocblas_handle rb = nullptr;  // made by the first eigensolve
     double* eri = nullptr;  // nBas^4 AO integrals (QuAcK's ERI.bin order)
     // nBas x nBas: S, P, F and three products; nBas x nOrb: X, c, c2, SC, T;
-    // nOrb x nOrb: Sig, Fp; w: nOrb; work: the eigensolve's
+    // nOrb x nOrb: Sig, Fp; w, work: nOrb
     double *S = nullptr, *P = nullptr, *F = nullptr, *A1 = nullptr, *A2 = nullptr, *A3 = nullptr;
     double *X = nullptr, *c = nullptr, *c2 = nullptr, *SC = nullptr, *Tm = nullptr;
     double *Sig = nullptr, *Fp = nullptr, *w = nullptr, *work = nullptr;
@@ -37,10 +38,12 @@ void qsgw_release(qk_qsgw_ctx* h) {
     dfree(h->info);
     if (h->g) (void)qk_gw_destroy(h->g);
     if (h->jk) (void)qk_rhf_destroy(h->jk);
+    if (h->rb) (void)rocblas_destroy_handle(h->rb);
     if (h->s) (void)hipStreamDestroy(h->s);
     delete h->diis;
     h->g = nullptr;
     h->jk = nullptr;
+    h->rb = nullptr;
     h->s = nullptr;
     h->diis = nullptr;
 }
@@ -88,12 +91,13 @@ int qk_qsgw_create(qk_qsgw_handle* out, int nBas, int nOrb, int nC, int nO, int 
         QK_CHECK(r == QK_OK, r, "qsGW: Hartree/exchange builder for nBas = " + std::to_string(nBas));
         r = qk_gw_create(&h->g, nBas, nOrb, nC, nO, nV, nR, nS);
         QK_CHECK(r == QK_OK, r, "qsGW: GW engine: " + std::string(qk_last_error()));
+        h->g->keep_syevd = true;
         h->eri = dalloc<double>(N2 * N2);
         for (double** p : {&h->S, &h->P, &h->F, &h->A1, &h->A2, &h->A3}) *p = dalloc<double>(N2);
         for (double** p : {&h->X, &h->c, &h->c2, &h->SC, &h->Tm}) *p = dalloc<double>(N * n);
         for (double** p : {&h->Sig, &h->Fp}) *p = dalloc<double>(n * n);
         h->w = dalloc<double>(n);
-        h->work = dalloc<double>(eigh_work_doubles((int)n, 1, true));
+        h->work = dalloc<double>(n);
         h->info = dalloc<int>(1);
         up(h->s, h->eri, ERI_AO, N2 * N2);
         up(h->s, h->S, S, N2);
@@ -200,7 +204,7 @@ int qk_qsgw_cycle(qk_qsgw_handle h, double eta, int TDA_W, int doSRG, double* eG
         const double* B = N == n ? h->X : h->c;
         dgemm(s, false, false, N, n, N, 1.0, h->F, N, B, N, 0.0, h->Tm, N);
         dgemm(s, true, false, n, n, N, 1.0, B, N, h->Tm, N, 0.0, h->Fp, n);
-        eigh_checked(s, n, h->Fp, h->w, true, h->work, h->info);
+        syevd(s, blas(h->rb, s), n, h->Fp, h->w, h->work, h->info);
         dgemm(s, false, false, N, n, n, 1.0, B, N, h->Fp, n, 0.0, h->c2, N);
         std::swap(h->c, h->c2);
         // SigC in the new orbitals (:335) and the density (:339)
