@@ -21,6 +21,8 @@ struct qk_gwb_ctx {
     int *info = nullptr, *active = nullptr, *nit = nullptr, *done = nullptr;
     double* eigw = nullptr;  // work of the eigensolves, on first use
     size_t eigw_doubles = 0;
+    double* aow = nullptr;  // work of aotomo_block, on first use
+    size_t aow_doubles = 0;
     qk::Zs zs;
     int nchunk = 1;
     // evGW state on the device (qk_gwb_evgw): DIIS histories, per molecule
@@ -65,7 +67,7 @@ void release_batch(BCtx* b) {
     }
     b->mol.clear();
     for (double* p : {b->M, b->Cm, b->rhoT, b->Om, b->E, b->K, b->dE, b->sd, b->Om0, b->part, b->scal, b->hist, b->conv,
-                      b->outSig, b->outZ, b->outOm, b->outEc, b->eigw})
+                      b->outSig, b->outZ, b->outOm, b->outEc, b->eigw, b->aow})
         if (p) (void)hipFree(p);
     for (double* p : b->vec)
         if (p) (void)hipFree(p);
@@ -359,8 +361,12 @@ int qk_gwb_set_eri_ao_device(qk_gwb_handle h, const double* ERI_AO, long long st
         const bool sp = split_aotomo();
         for (int m = 0; m < h->nmol; ++m) {
             Ctx* x = h->mol[m];
+            // one molecule after the other on the stream: they share the buffer
+            AoScratch w;
+            if (!sp)
+                w = ao_scratch(x->nBas, x->nOrb, x->nC, x->nO, x->nR, x->nS, h->aow, h->aow_doubles, x->rhoT);
             aotomo_block(h->s, ERI_AO + m * stride_eri, c + m * stride_c, x->M, x->nBas, x->nOrb, x->nC, x->nO,
-                         x->nR, sp, x->K);
+                         x->nR, sp, x->K, w.t1, w.t2);
             if (!sp) extract_k(h->s, x->M, x->K, x->nOrb, x->nC, x->nO, x->v, x->nS);
             x->msplit_valid = false;
             x->have_eri = true;

@@ -156,6 +156,8 @@ struct qk_gw_ctx {
     bool keep_syevd = false;  // qsGW's engine: eigenvectors from rocSOLVER dsyevd
     double* eigw = nullptr;   // work of the full solves, on first use
     size_t eigw_doubles = 0;
+    double* aow = nullptr;  // work of aotomo_block, on first use
+    size_t aow_doubles = 0;
     double *Zev = nullptr, *tau = nullptr, *trd_work = nullptr, *orm_work = nullptr;  // split-precision full solves
     qk::SolveGraphs graphs;  // captured launch sequences of the own full solve
     double *Xv = nullptr, *Ym = nullptr, *Sm = nullptr, *Gm = nullptr, *lam = nullptr, *eig_dbuf = nullptr;
@@ -204,7 +206,12 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
 // split-precision AO->MO block switch (qk_set_split_aotomo)
 bool split_aotomo();
 void aotomo_block(hipStream_t s, const double* f, const double* cc, double* M, int N, int n, int nC, int nO, int nR,
-                  bool split = false, double* K = nullptr);
+                  bool split = false, double* K = nullptr, double* work1 = nullptr, double* work2 = nullptr);
+// its two work arrays for a handle (null: it allocates); buf, cap: the handle's kept buffer
+struct AoScratch {
+    double *t1 = nullptr, *t2 = nullptr;
+};
+AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf, size_t& cap, double* rhoT);
 void upload_mo_block(hipStream_t s, const double* ERI_MO, double* M, int n, int nC, int nO, int nR);
 // rho(p,q,m) (QuAcK layout, host) into rhoT[m + nS (p + n q)] on the device (caller frees)
 double* upload_rho(hipStream_t s, const double* rho, int n, int nS);
