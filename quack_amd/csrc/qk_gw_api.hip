@@ -11,6 +11,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <memory>
 
 #include "qk_gw_internal.h"
 
@@ -26,12 +27,14 @@ void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double
     QK_CHECK(info == 0, QK_E_EIG, "rocsolver_dsyevd failed, info = " + std::to_string(info));
 }
 
+const char* const NOT_FINITE = "eigensolver: the matrix has entries that are not finite";
+
 void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, hipEvent_t* tev) {
     eigh(s, n, 1, A, (long long)n * n, w, n, vectors, work, dinfo, tev);
     int info = 0;
     QK_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
     QK_HIP(hipStreamSynchronize(s));
-    QK_CHECK(info == 0, QK_E_EIG, "eigensolver: the matrix has entries that are not finite");
+    QK_CHECK(info == 0, QK_E_EIG, NOT_FINITE);
 }
 
 // Tiny symmetric solve for DIIS: LU with partial pivoting; rcond is the exact
@@ -874,6 +877,123 @@ AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf,
     return r;
 }
 
+// LR/phRLR.f90 for a number of problems of one order side by side on the device: the
+// caller fills A and B (S2 apart), solve() leaves Om in w, EcRPA in sc[4 m + 1] and,
+// with vectors, X + Y in ApB and X - Y in B (A and B under TDA: X in B).
+// Both eigensolves are one launch chain for all problems, and those that nobody asks
+// eigenvectors of are values only: singlet and triplet BSE of N = 60 (nS = 324) cost two
+// tridiagonalisations, 1.5 ms, where one spin after the other took four, 3.0 ms.
+struct PhRlr {
+    hipStream_t s;
+    int nS, batch, tda;
+    bool vectors;
+    size_t S2;
+    double *A = nullptr, *B = nullptr, *U = nullptr, *ApB = nullptr, *T = nullptr, *Ti = nullptr;
+    double *w = nullptr, *work = nullptr, *sc = nullptr;
+    int* info = nullptr;
+    Error err{QK_OK, ""};  // of the first problem that failed
+    PhRlr(hipStream_t s_, int nS_, int batch_, int tda_, bool vec)
+        : s(s_), nS(nS_), batch(batch_), tda(tda_), vectors(vec), S2((size_t)nS_ * nS_) {
+        try {
+            A = dalloc<double>(S2 * batch);
+            U = dalloc<double>(S2 * batch);
+            if (!tda || vectors) B = dalloc<double>(S2 * batch);
+            if (!tda) {
+                ApB = dalloc<double>(S2 * batch);
+                T = dalloc<double>(S2 * batch);
+                if (vectors) Ti = dalloc<double>(S2 * batch);
+            }
+            w = dalloc<double>((size_t)nS * batch);
+            work = dalloc<double>(eigh_work_doubles(nS, batch, vectors || !tda));
+            sc = dalloc<double>(4 * (size_t)batch);
+            info = dalloc<int>(batch);
+        } catch (...) {
+            release();
+            throw;
+        }
+    }
+    PhRlr(const PhRlr&) = delete;
+    PhRlr& operator=(const PhRlr&) = delete;
+    ~PhRlr() { release(); }
+    void release() {
+        (void)hipStreamSynchronize(s);
+        for (double** p : {&A, &B, &U, &ApB, &T, &Ti, &w, &work, &sc}) dfree(*p);
+        dfree(info);
+    }
+    // the eigensolve of the first nb matrices in U; returns how many of them stand
+    int eig(int nb, bool vec, bool positive) {
+        eigh(s, nS, nb, U, (long long)S2, w, nS, vec, work, info);
+        std::vector<int> bad(nb);
+        std::vector<double> low(nb);
+        QK_HIP(hipMemcpyAsync(bad.data(), info, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
+        if (positive)
+            for (int m = 0; m < nb; ++m)
+                QK_HIP(hipMemcpyAsync(&low[m], w + (size_t)nS * m, sizeof(double), hipMemcpyDeviceToHost, s));
+        QK_HIP(hipStreamSynchronize(s));
+        for (int m = 0; m < nb; ++m) {
+            if (bad[m] != 0) {
+                err = Error{QK_E_EIG, NOT_FINITE};
+                return m;
+            }
+            // LR/phRLR.f90:57-58: QuAcK warns when A - B has a negative
+            // eigenvalue and then takes its square root; stop before the
+            // NaN (or the infinite inverse root of a zero mode) spreads
+            if (positive && !(low[m] > 0.0)) {
+                err = Error{QK_E_UNSTABLE, "phRLR: A-B is not positive definite (smallest eigenvalue " +
+                                               std::to_string(low[m]) + "): linear-response instability"};
+                return m;
+            }
+        }
+        return nb;
+    }
+    // returns the number of leading problems that are solved (batch, or err tells why not)
+    int solve() {
+        int nb = batch;
+        Zs zs;
+        zs.S = nS;
+        zs.c = 4;
+        for (int m = 0; m < nb; ++m) trace(s, A + S2 * m, nS, sc + 4 * m);
+        if (tda) {
+            // LR/phRLR.f90:40-43
+            QK_HIP(hipMemcpyAsync(U, A, sizeof(double) * S2 * nb, hipMemcpyDeviceToDevice, s));
+            nb = eig(nb, vectors, false);
+            if (vectors)
+                for (int m = 0; m < nb; ++m) transpose(s, U + S2 * m, B + S2 * m, nS, nS, nS, nS);
+            if (nb > 0) rpa_finalize(s, w, nullptr, nullptr, sc, nS, 1, false, zs, nb);
+            return nb;
+        }
+        // LR/phRLR.f90:47-81 with A - B = U d U^T in its eigenvectors' basis:
+        // T = U d^1/2, Z = T^T (A + B) T, (X + Y)^T = T V Om^-1/2, (X - Y)^T = U d^-1/2 V Om^1/2
+        apb_amb(s, A, B, ApB, U, (long long)(S2 * nb));
+        nb = eig(nb, true, true);
+        if (nb == 0) return 0;
+        for (int m = 0; m < nb; ++m) {
+            colscale_pow(s, U + S2 * m, w + (size_t)nS * m, T + S2 * m, nS, 0.5);
+            if (vectors) colscale_pow(s, U + S2 * m, w + (size_t)nS * m, Ti + S2 * m, nS, -0.5);
+        }
+        Batch b;
+        b.zdiv = b.count = nb;
+        b.sa0 = b.sb0 = b.sc0 = (long long)S2;
+        dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, T, nS, 0.0, A, nS, b);
+        dgemm(s, true, false, nS, nS, nS, 1.0, T, nS, A, nS, 0.0, U, nS, b);
+        nb = eig(nb, vectors, false);
+        if (nb == 0) return 0;
+        b.zdiv = b.count = nb;
+        rpa_finalize(s, w, nullptr, nullptr, sc, nS, 0, false, zs, nb);  // Om = sqrt|w|
+        if (vectors) {
+            dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, T, nS, 0.0, ApB, nS, b);
+            dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, Ti, nS, 0.0, B, nS, b);
+            for (int m = 0; m < nb; ++m) {
+                rowscale_pow(s, ApB + S2 * m, w + (size_t)nS * m, nS, -0.5);
+                rowscale_pow(s, B + S2 * m, w + (size_t)nS * m, nS, 0.5);
+            }
+        }
+        return nb;
+    }
+    const double* xpy() const { return tda ? B : ApB; }
+    const double* xmy() const { return B; }
+};
+
 // The four-index block M is allocated on first use (a density-fitted handle never needs it).
 void ensure_m(Ctx* c) {
     if (!c->M) c->M = dalloc<double>((size_t)c->nOrb * c->nOrb * c->nS);
@@ -1510,73 +1630,17 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
     if (nS <= 0 || !Aph || (!TDA && !Bph) || !Om || !XpY || !XmY) return QK_E_ARG;
     return guarded(nullptr, [&] {
         hipStream_t s = scratch().s;
-        size_t S2 = (size_t)nS * nS;
-        std::vector<double*> bufs;
-        auto get = [&](size_t cnt) { bufs.push_back(dalloc<double>(cnt)); return bufs.back(); };
-        try {
-            double* A = get(S2);
-            double* U = get(S2);
-            double* w = get(nS);
-            double* work = get(eigh_work_doubles(nS, 1, true));
-            double* sc = get(4);
-            int* info = dalloc<int>(1);
-            bufs.push_back(reinterpret_cast<double*>(info));
-            QK_HIP(hipMemcpyAsync(A, Aph, sizeof(double) * S2, hipMemcpyHostToDevice, s));
-            trace(s, A, nS, sc);
-            if (TDA) {
-                // LR/phRLR.f90:40-43
-                QK_HIP(hipMemcpyAsync(U, A, sizeof(double) * S2, hipMemcpyDeviceToDevice, s));
-                eigh_checked(s, nS, U, w, true, work, info);
-                double* X = get(S2);
-                transpose(s, U, X, nS, nS, nS, nS);
-                rpa_finalize(s, w, nullptr, nullptr, sc, nS, 1, false);
-                QK_HIP(hipMemcpyAsync(XpY, X, sizeof(double) * S2, hipMemcpyDeviceToHost, s));
-                QK_HIP(hipMemcpyAsync(XmY, X, sizeof(double) * S2, hipMemcpyDeviceToHost, s));
-            } else {
-                // LR/phRLR.f90:47-81
-                double* B = get(S2);
-                double* ApB = get(S2);
-                double* Sq = get(S2);
-                double* Iv = get(S2);
-                double* T = get(S2);
-                QK_HIP(hipMemcpyAsync(B, Bph, sizeof(double) * S2, hipMemcpyHostToDevice, s));
-                apb_amb(s, A, B, ApB, U, (long long)S2);
-                eigh_checked(s, nS, U, w, true, work, info);
-                // LR/phRLR.f90:57-58: QuAcK warns when A - B has a negative
-                // eigenvalue and then takes its square root; stop before the
-                // NaN (or the infinite inverse root of a zero mode) spreads
-                double wmin = 0.0;
-                QK_HIP(hipMemcpyAsync(&wmin, w, sizeof(double), hipMemcpyDeviceToHost, s));
-                QK_HIP(hipStreamSynchronize(s));
-                QK_CHECK(wmin > 0.0, QK_E_UNSTABLE,
-                         "phRLR: A-B is not positive definite (smallest eigenvalue " + std::to_string(wmin) +
-                             "): linear-response instability");
-                colscale_pow(s, U, w, T, nS, 0.5);
-                dgemm(s, false, true, nS, nS, nS, 1.0, T, nS, U, nS, 0.0, Sq, nS);   // ADAt(U, sqrt(w))
-                colscale_pow(s, U, w, T, nS, -0.5);
-                dgemm(s, false, true, nS, nS, nS, 1.0, T, nS, U, nS, 0.0, Iv, nS);   // ADAt(U, 1/sqrt(w))
-                dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, Sq, nS, 0.0, T, nS);  // tmp = ApB AmBSq
-                dgemm(s, false, false, nS, nS, nS, 1.0, Sq, nS, T, nS, 0.0, U, nS);    // Z = AmBSq tmp
-                eigh_checked(s, nS, U, w, true, work, info);
-                rpa_finalize(s, w, nullptr, nullptr, sc, nS, 0, false);                 // Om = sqrt|w|
-                dgemm(s, true, false, nS, nS, nS, 1.0, U, nS, Sq, nS, 0.0, T, nS);     // XpY = Z^T AmBSq
-                rowscale_pow(s, T, w, nS, -0.5);
-                QK_HIP(hipMemcpyAsync(XpY, T, sizeof(double) * S2, hipMemcpyDeviceToHost, s));
-                dgemm(s, true, false, nS, nS, nS, 1.0, U, nS, Iv, nS, 0.0, ApB, nS);   // XmY = Z^T AmBIv
-                rowscale_pow(s, ApB, w, nS, 0.5);
-                QK_HIP(hipMemcpyAsync(XmY, ApB, sizeof(double) * S2, hipMemcpyDeviceToHost, s));
-            }
-            QK_HIP(hipMemcpyAsync(Om, w, sizeof(double) * nS, hipMemcpyDeviceToHost, s));
-            double ec = 0.0;
-            QK_HIP(hipMemcpyAsync(&ec, sc + 1, sizeof(double), hipMemcpyDeviceToHost, s));
-            QK_HIP(hipStreamSynchronize(s));
-            if (EcRPA) *EcRPA = ec;
-        } catch (...) {
-            (void)hipStreamSynchronize(s);
-            for (double* p : bufs) (void)hipFree(p);
-            throw;
-        }
-        for (double* p : bufs) (void)hipFree(p);
+        PhRlr r(s, nS, 1, TDA, true);
+        QK_HIP(hipMemcpyAsync(r.A, Aph, sizeof(double) * r.S2, hipMemcpyHostToDevice, s));
+        if (!TDA) QK_HIP(hipMemcpyAsync(r.B, Bph, sizeof(double) * r.S2, hipMemcpyHostToDevice, s));
+        if (r.solve() != 1) throw r.err;
+        double ec = 0.0;
+        QK_HIP(hipMemcpyAsync(XpY, r.xpy(), sizeof(double) * r.S2, hipMemcpyDeviceToHost, s));
+        QK_HIP(hipMemcpyAsync(XmY, r.xmy(), sizeof(double) * r.S2, hipMemcpyDeviceToHost, s));
+        QK_HIP(hipMemcpyAsync(Om, r.w, sizeof(double) * nS, hipMemcpyDeviceToHost, s));
+        QK_HIP(hipMemcpyAsync(&ec, r.sc + 1, sizeof(double), hipMemcpyDeviceToHost, s));
+        QK_HIP(hipStreamSynchronize(s));
+        if (EcRPA) *EcRPA = ec;
     });
 }
 
@@ -1646,62 +1710,45 @@ int qk_rgw_phbse_dyn(int dophBSE2, int exchange_kernel, int TDA_W, int TDA, int 
         // matrix-core products over the RPA modes m:
         //   KA(ia,jb) = 4 sum_m [w_m rho(i,j,m)] rho(a,b,m) -> G1[(i + o j), (a + v b)]
         //   KB(ia,jb) = 4 sum_m [w_m rho(i,b,m)] rho(a,j,m) -> G2[(i + o b), (a + v j)]
-        std::vector<double> KA(S2, 0.0), KB(S2, 0.0);
+        std::vector<double> KA, KB;           // the kernels on the host, for dBSE
+        double *G1 = nullptr, *G2 = nullptr;  // freed by free_extra
+        // device buffers of the second-order kernel and the dynamical correction
+        double *dW = nullptr, *dE = nullptr, *dX = nullptr, *dY = nullptr, *dPart = nullptr, *dK = nullptr;
+        double *dD = nullptr, *dKs = nullptr;
+        auto free_extra = [&] {
+            (void)hipStreamSynchronize(c->s);
+            for (double** p : {&G1, &G2, &dW, &dE, &dX, &dY, &dPart, &dK, &dD, &dKs}) dfree(*p);
+        };
+        try {
         {
             double* X = dalloc<double>((size_t)nS * o * std::max(o, v));
             double* Y = nullptr;
-            double* G = nullptr;
             try {
                 Y = dalloc<double>((size_t)nS * v * std::max(o, v));
-                G = dalloc<double>(S2 > (size_t)o * o * v * v ? S2 : (size_t)o * o * v * v);
-                std::vector<double> hG((size_t)o * o * v * v);
+                G1 = dalloc<double>((size_t)o * o * v * v);
                 rho_block(c->s, c->rhoT, c->Om, eta, 1, n, nS, nC, o, nC, o, X);
                 rho_block(c->s, c->rhoT, c->Om, eta, 0, n, nS, nO, v, nO, v, Y);
-                dgemm(c->s, true, false, o * o, v * v, nS, 1.0, X, nS, Y, nS, 0.0, G, o * o);
-                QK_HIP(hipMemcpyAsync(hG.data(), G, sizeof(double) * hG.size(), hipMemcpyDeviceToHost, c->s));
-                QK_HIP(hipStreamSynchronize(c->s));
-                for (int i = 0; i < o; ++i)
-                    for (int a = 0; a < v; ++a)
-                        for (int j = 0; j < o; ++j)
-                            for (int b = 0; b < v; ++b)
-                                KA[(a + (size_t)v * i) + nS * (b + (size_t)v * j)] =
-                                    4.0 * hG[(i + (size_t)o * j) + (size_t)o * o * (a + (size_t)v * b)];
+                dgemm(c->s, true, false, o * o, v * v, nS, 1.0, X, nS, Y, nS, 0.0, G1, o * o);
                 if (!TDA) {
+                    G2 = dalloc<double>(S2);
                     rho_block(c->s, c->rhoT, c->Om, eta, 1, n, nS, nC, o, nO, v, X);
                     rho_block(c->s, c->rhoT, c->Om, eta, 0, n, nS, nO, v, nC, o, Y);
-                    dgemm(c->s, true, false, o * v, v * o, nS, 1.0, X, nS, Y, nS, 0.0, G, o * v);
-                    hG.resize(S2);
-                    QK_HIP(hipMemcpyAsync(hG.data(), G, sizeof(double) * S2, hipMemcpyDeviceToHost, c->s));
-                    QK_HIP(hipStreamSynchronize(c->s));
-                    for (int i = 0; i < o; ++i)
-                        for (int a = 0; a < v; ++a)
-                            for (int j = 0; j < o; ++j)
-                                for (int b = 0; b < v; ++b)
-                                    KB[(a + (size_t)v * i) + nS * (b + (size_t)v * j)] =
-                                        4.0 * hG[(i + (size_t)o * b) + (size_t)o * v * (a + (size_t)v * j)];
+                    dgemm(c->s, true, false, o * v, v * o, nS, 1.0, X, nS, Y, nS, 0.0, G2, o * v);
                 }
             } catch (...) {
                 (void)hipStreamSynchronize(c->s);
-                dfree(X); dfree(Y); dfree(G);
+                dfree(X); dfree(Y);
                 throw;
             }
-            dfree(X); dfree(Y); dfree(G);
+            QK_HIP(hipStreamSynchronize(c->s));
+            dfree(X); dfree(Y);
         }
-        auto G = [&](int p, int q, int r, int t) {  // ERI(p,q,r,s), 0-based
+        auto G = [&](int p, int q, int r, int t) -> const double& {  // ERI(p,q,r,s), 0-based
             return ERI[p + (size_t)n * (q + (size_t)n * (r + (size_t)n * t))];
         };
-        // device buffers of the second-order kernel and the dynamical correction
-        double *dW = nullptr, *dE = nullptr, *dX = nullptr, *dY = nullptr, *dPart = nullptr, *dK = nullptr;
-        auto free_extra = [&] {
-            (void)hipStreamSynchronize(c->s);
-            dfree(dW); dfree(dE); dfree(dX); dfree(dY); dfree(dPart); dfree(dK);
-        };
-        try {
-        if (dophBSE2 || dBSE) {
-            dE = dalloc<double>(2 * (size_t)n);  // eW, then eGW
-            QK_HIP(hipMemcpyAsync(dE, eW, sizeof(double) * n, hipMemcpyHostToDevice, c->s));
-            QK_HIP(hipMemcpyAsync(dE + n, eGW, sizeof(double) * n, hipMemcpyHostToDevice, c->s));
-        }
+        dE = dalloc<double>(2 * (size_t)n);  // eW, then eGW
+        QK_HIP(hipMemcpyAsync(dE, eW, sizeof(double) * n, hipMemcpyHostToDevice, c->s));
+        QK_HIP(hipMemcpyAsync(dE + n, eGW, sizeof(double) * n, hipMemcpyHostToDevice, c->s));
         if (dophBSE2) {
             // GW/RGW_phBSE_static_kernel.f90:40-60: W(p,s,q,r) = -ERI(p,s,q,r) + 4 chi(pq, rs),
             // chi = sum_m rho(p,q,m) w_m rho(r,s,m) as one FP64 matrix-core product
@@ -1739,48 +1786,62 @@ int qk_rgw_phbse_dyn(int dophBSE2, int exchange_kernel, int TDA_W, int TDA, int 
         }
         // singlet (ispin 1) and triplet (ispin 2): phRLR_A/B with dRPA = false at
         // eGW (LR/phRLR_A.f90:43-115, LR/phRLR_B.f90:34-95) plus the kernels,
-        // then phRLR (GW/RGW_phBSE.f90:133-190)
-        std::vector<double> A(S2), B(S2), XpY(S2), XmY(S2);
+        // then phRLR (GW/RGW_phBSE.f90:133-190), both spins side by side
         for (int k = 0; k < 2 * nS; ++k) OmBSE[k] = 0.0;
         EcBSE[0] = EcBSE[1] = 0.0;
-        for (int ispin = 1; ispin <= 2; ++ispin) {
-            if ((ispin == 1 && !singlet) || (ispin == 2 && !triplet)) continue;
-            if (ispin == 1 && dophBSE2) {
-                // GW/RGW_phBSE.f90:123-138: the second-order kernels are added onto
-                // KA/KB (the BSE2 routines accumulate into the array RGW_phBSE
-                // passes, which holds the first-order kernel); the triplet
-                // block after this one uses the kernels so changed
-                dK = dalloc<double>(2 * S2);
-                bse2_static(c->s, dW, dE, eta, n, nO, nS, dK, TDA ? nullptr : dK + S2);
-                std::vector<double> h(2 * S2);
-                QK_HIP(hipMemcpyAsync(h.data(), dK, sizeof(double) * (TDA ? S2 : 2 * S2), hipMemcpyDeviceToHost,
-                                      c->s));
-                QK_HIP(hipStreamSynchronize(c->s));
-                for (size_t k = 0; k < S2; ++k) KA[k] += h[k];
-                if (!TDA)
-                    for (size_t k = 0; k < S2; ++k) KB[k] += h[S2 + k];
-                dfree(dK);
-            }
-            const double ct1 = ispin == 1 ? 2.0 : 0.0, ct2 = -1.0;
+        const int spins = (singlet ? 1 : 0) + (triplet ? 2 : 0), nspin = (singlet ? 1 : 0) + (triplet ? 1 : 0);
+        if (singlet && dophBSE2) {
+            // GW/RGW_phBSE.f90:123-138: the second-order kernels are added onto
+            // KA/KB (the BSE2 routines accumulate into the array RGW_phBSE
+            // passes, which holds the first-order kernel) in the singlet block;
+            // the triplet block after it uses the kernels so changed
+            dK = dalloc<double>(2 * S2);
+            bse2_static(c->s, dW, dE, eta, n, nO, nS, dK, TDA ? nullptr : dK + S2);
+        }
+        std::unique_ptr<PhRlr> lr;
+        int solved = 0;
+        if (nspin > 0) {
+            lr.reset(new PhRlr(c->s, nS, nspin, TDA, dBSE != 0));
+            // the integrals of A and B: D1(b,i,j,a) = ERI(b,i,j,a), D2(b,j,a,i) = ERI(b,j,a,i)
+            std::vector<double> hD(2 * S2);
+            double *D1 = hD.data(), *D2 = D1 + S2;
+            for (int a = 0; a < v; ++a)
+                for (int j = 0; j < o; ++j)
+                    for (int i = 0; i < o; ++i, D1 += v)
+                        std::memcpy(D1, &G(nO, nC + i, nC + j, nO + a), sizeof(double) * v);
             for (int i = 0; i < o; ++i)
-                for (int a = 0; a < v; ++a) {
-                    const size_t ia = a + (size_t)v * i;
-                    const int I = nC + i, Aa = nO + a;
-                    for (int j = 0; j < o; ++j)
-                        for (int b = 0; b < v; ++b) {
-                            const size_t jb = b + (size_t)v * j;
-                            const int J = nC + j, Bb = nO + b;
-                            const double d = G(Bb, I, J, Aa);
-                            double aij = ct1 * d + ct2 * G(Bb, J, Aa, I) + KA[ia + nS * jb];
-                            if (i == j && a == b) aij += eGW[Aa] - eGW[I];
-                            A[ia + nS * jb] = aij;
-                            B[ia + nS * jb] = TDA ? 0.0 : ct1 * d + ct2 * G(Bb, J, I, Aa) + KB[ia + nS * jb];
-                        }
-                }
+                for (int a = 0; a < v; ++a)
+                    for (int j = 0; j < o; ++j, D2 += v)
+                        std::memcpy(D2, &G(nO, nC + j, nO + a, nC + i), sizeof(double) * v);
+            dD = dalloc<double>(2 * S2);
+            QK_HIP(hipMemcpyAsync(dD, hD.data(), sizeof(double) * 2 * S2, hipMemcpyHostToDevice, c->s));
+            if (dBSE) dKs = dalloc<double>(2 * S2);
+            bse_ab(c->s, dD, G1, G2, dK, dE + n, nC, nO, o, v, spins, lr->A, TDA ? nullptr : lr->B, dKs);
+            if (dBSE) {
+                KA.resize(S2);
+                KB.resize(S2);
+                QK_HIP(hipMemcpyAsync(KA.data(), dKs, sizeof(double) * S2, hipMemcpyDeviceToHost, c->s));
+                QK_HIP(hipMemcpyAsync(KB.data(), dKs + S2, sizeof(double) * S2, hipMemcpyDeviceToHost, c->s));
+            }
+            QK_HIP(hipStreamSynchronize(c->s));  // hD
+            solved = lr->solve();
+        }
+        std::vector<double> XpY(dBSE ? S2 : 0), XmY(dBSE ? S2 : 0);
+        for (int ispin = 1, k = 0; ispin <= 2; ++ispin) {
+            if ((ispin == 1 && !singlet) || (ispin == 2 && !triplet)) continue;
+            QK_CHECK(k < solved, lr->err.code, "qk_rgw_phbse: phRLR failed: " + lr->err.msg);
             double ec = 0.0;
             double* Om = OmBSE + (size_t)(ispin - 1) * nS;
-            const int r = qk_phrlr(TDA, nS, A.data(), B.data(), &ec, Om, XpY.data(), XmY.data());
-            QK_CHECK(r == QK_OK, r, "qk_rgw_phbse: phRLR failed: " + g_last_error);
+            QK_HIP(hipMemcpyAsync(Om, lr->w + (size_t)nS * k, sizeof(double) * nS, hipMemcpyDeviceToHost, c->s));
+            QK_HIP(hipMemcpyAsync(&ec, lr->sc + 4 * k + 1, sizeof(double), hipMemcpyDeviceToHost, c->s));
+            if (dBSE) {
+                QK_HIP(hipMemcpyAsync(XpY.data(), lr->xpy() + S2 * k, sizeof(double) * S2, hipMemcpyDeviceToHost,
+                                      c->s));
+                QK_HIP(hipMemcpyAsync(XmY.data(), lr->xmy() + S2 * k, sizeof(double) * S2, hipMemcpyDeviceToHost,
+                                      c->s));
+            }
+            QK_HIP(hipStreamSynchronize(c->s));
+            ++k;
             EcBSE[ispin - 1] = ec;
             if (!dBSE) continue;
             // GW/RGW_phBSE_dynamic_perturbation.f90:73-122 for the first

@@ -62,6 +62,45 @@ __global__ void k_bse2_static(const double* __restrict__ Wp, const double* __res
     if (KB2) KB2[t] = kb;
 }
 
+// LR/phRLR_A.f90:43-115 and LR/phRLR_B.f90:34-95 with dRPA = false at e = eGW plus the
+// static kernels KA(ia,jb) = 4 G1, KB(ia,jb) = 4 G2 (+ second order), for the spins asked
+// for: every operand is read once for both.  One thread an element, A's column along the
+// wave: the stores are whole lines and the permuted operands (0.8 MB each at nS = 324)
+// come from L2.  Built by host loops, with the kernels brought back and A and B sent over
+// for each spin, this took 3 ms of a call of 14.5 ms at nS = 324.
+__global__ void k_bse_ab(const double* __restrict__ D, const double* __restrict__ G1, const double* __restrict__ G2,
+                         const double* __restrict__ K2, const double* __restrict__ e, int nC, int nO, int o, int v,
+                         int spins, double* __restrict__ A, double* __restrict__ B, double* __restrict__ Ks) {
+    const long long nS = (long long)o * v, S2 = nS * nS;
+    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (t >= S2) return;
+    const int ia = (int)(t % nS), jb = (int)(t / nS);
+    const int a = ia % v, i = ia / v, b = jb % v, j = jb / v;
+    const double d = D[b + v * (i + o * (j + (long long)o * a))];
+    const double xa = D[S2 + b + v * (j + o * (a + (long long)v * i))];
+    double ka = 4.0 * G1[(i + o * j) + (long long)o * o * (a + (long long)v * b)], kb = 0.0;
+    if (K2) ka += K2[t];
+    const double gap = ia == jb ? e[nO + a] - e[nC + i] : 0.0;
+    double xb = 0.0;
+    if (B) {
+        xb = D[b + v * (j + o * (i + (long long)o * a))];
+        kb = 4.0 * G2[(i + o * b) + nS * (a + (long long)v * j)];
+        if (K2) kb += K2[S2 + t];
+    }
+    long long to = t;
+    for (int sp = 0; sp < 2; ++sp) {
+        if (!(spins >> sp & 1)) continue;
+        const double c = sp == 0 ? 2.0 : 0.0;
+        A[to] = c * d - xa + ka + gap;
+        if (B) B[to] = c * d - xb + kb;
+        to += S2;
+    }
+    if (Ks) {
+        Ks[t] = ka;
+        Ks[S2 + t] = kb;
+    }
+}
+
 // The six quadratic forms of GW/RGW_phBSE_dynamic_perturbation.f90:86-112 for
 // one BSE excitation Om with vectors X, Y: per element (ia, jb) the dynamic
 // kernels KA(+Om), ZA(+Om) (GW/RGW_phBSE_dynamic_kernel_A.f90:38-82, plus the
@@ -171,6 +210,14 @@ void bse2_static(hipStream_t s, const double* W, const double* e, double eta, in
     const long long tot = (long long)nS * nS;
     hipLaunchKernelGGL(k_bse2_static, dim3((unsigned)((tot + TB - 1) / TB)), dim3(TB), 0, s, W, e, eta, n, nO, nS,
                        KA2, KB2);
+    QK_HIP(hipGetLastError());
+}
+
+void bse_ab(hipStream_t s, const double* D, const double* G1, const double* G2, const double* K2, const double* e,
+            int nC, int nO, int o, int v, int spins, double* A, double* B, double* Ks) {
+    const long long nS = (long long)o * v;
+    hipLaunchKernelGGL(k_bse_ab, dim3((unsigned)((nS * nS + TB - 1) / TB)), dim3(TB), 0, s, D, G1, G2, K2, e, nC, nO, o,
+                       v, spins, A, B, Ks);
     QK_HIP(hipGetLastError());
 }
 

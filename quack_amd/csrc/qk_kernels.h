@@ -73,6 +73,12 @@ void rho_block(hipStream_t s, const double* rhoT, const double* Om, double eta, 
 // from the 4-index W of GW/RGW_phBSE_static_kernel.f90 (KB2 skipped when null).
 void bse2_static(hipStream_t s, const double* W, const double* e, double eta, int n, int nO, int nS, double* KA2,
                  double* KB2);
+// A and B (null under TDA) of the singlet and/or triplet BSE (spins: bit 0, bit 1; each
+// nS x nS, one after the other) from D1(b,i,j,a) and behind it D2(b,j,a,i), the kernel
+// products G1[(i + o j) + o^2 (a + v b)], G2[(i + o b) + o v (a + v j)] (null: none) and the
+// second-order kernels K2 (KA2, then KB2; null: none); Ks (or null): KA, then KB.
+void bse_ab(hipStream_t s, const double* D, const double* G1, const double* G2, const double* K2, const double* e,
+            int nC, int nO, int o, int v, int spins, double* A, double* B, double* Ks);
 // The quadratic forms of the first-order dynamical BSE correction for one
 // excitation (GW/RGW_phBSE_dynamic_perturbation.f90): 6 partial sums per
 // block of bse_dyn_blocks(nS) blocks in part.
