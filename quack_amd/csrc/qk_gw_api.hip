@@ -1014,35 +1014,85 @@ void after_eri(Ctx* c, bool k_done = false) {
     c->have_eri = true;
 }
 
-// gather X[p + n j' + n o q + n o n b'] = ERI_MO(p, nC+j', q, nO+b') on the host
-void gather_mo_block(const double* ERI, double* X, int n, int nC, int nO, int nR) {
-    int o = nO - nC, v = n - nR - nO;
-    size_t n1 = n, n2 = n1 * n, n3 = n2 * n;
-    for (int b = 0; b < v; ++b)
-        for (int q = 0; q < n; ++q)
-            std::memcpy(X + n1 * o * (q + n1 * b), ERI + n1 * nC + n2 * q + n3 * (nO + b), sizeof(double) * n1 * o);
+RowUpload::RowUpload(hipStream_t s_, size_t longest, size_t total)
+    : s(s_), slot(std::min(std::max(longest, (size_t)1 << 16), total)) {
+    try {
+        QK_HIP(hipHostMalloc((void**)&h, SLOTS * slot * sizeof(double), hipHostMallocDefault));
+        for (hipEvent_t& e : ev) QK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } catch (...) {
+        release();
+        throw;
+    }
 }
 
+void RowUpload::release() {
+    (void)hipStreamSynchronize(s);
+    for (hipEvent_t e : ev)
+        if (e) (void)hipEventDestroy(e);
+    (void)hipHostFree(h);
+}
+
+void RowUpload::send(double* dst, size_t cnt) {
+    QK_HIP(hipMemcpyAsync(dst, h + turn % SLOTS * slot, cnt * sizeof(double), hipMemcpyHostToDevice, s));
+    QK_HIP(hipEventRecord(ev[turn % SLOTS], s));
+    if (++turn >= SLOTS) QK_HIP(hipEventSynchronize(ev[turn % SLOTS]));
+}
+
+void RowUpload::rows(double* dX, const double* base, size_t len, size_t n1, size_t s1, size_t n2, size_t s2, size_t n3,
+                     size_t s3) {
+    if (len == 0 || n1 * n2 * n3 == 0) return;
+    QK_CHECK(len <= slot, QK_E_ARG, "RowUpload: row longer than announced");
+    struct Walk {  // the rows in their order
+        const double* row;
+        size_t n1, s1, n2, s2, s3, i1, i2, i3;
+        void step() {
+            row += s1;
+            if (++i1 < n1) return;
+            i1 = 0;
+            row += s2 - n1 * s1;
+            if (++i2 < n2) return;
+            i2 = 0;
+            row += s3 - n2 * s2;
+            ++i3;
+        }
+    } at{base, n1, s1, n2, s2, s3, 0, 0, 0}, lead = at;
+    const size_t per = slot / len;
+    const auto fetch = [&] {
+        if (lead.i3 >= n3) return;
+        for (size_t k = 0; k < len; k += 8) __builtin_prefetch(lead.row + k);
+        lead.step();
+    };
+    for (size_t k = 0; k < 2 + 256 / len; ++k) fetch();
+    while (at.i3 < n3) {
+        double* d = h + turn % SLOTS * slot;
+        size_t fill = 0;
+        for (; fill < per && at.i3 < n3; ++fill, d += len, at.step()) {
+            fetch();
+            if (len < 16)
+                for (size_t k = 0; k < len; ++k) d[k] = at.row[k];
+            else
+                std::memcpy(d, at.row, len * sizeof(double));
+        }
+        send(dX, fill * len);
+        dX += fill * len;
+    }
+}
+
+// M of the active pairs from ERI_MO(p, nC+j', q, nO+b') on the host
 void upload_mo_block(hipStream_t s, const double* ERI_MO, double* M, int n, int nC, int nO, int nR) {
-    int o = nO - nC, v = n - nR - nO;
-    size_t cnt = (size_t)n * n * o * v;
-    double* hX = nullptr;
-    QK_HIP(hipHostMalloc((void**)&hX, cnt * sizeof(double), hipHostMallocDefault));
-    double* dX = nullptr;
+    const size_t o = nO - nC, v = n - nR - nO, n1 = n, n2 = n1 * n, n3 = n2 * n;
+    double* dX = dalloc<double>(n2 * o * v);
     try {
-        gather_mo_block(ERI_MO, hX, n, nC, nO, nR);
-        dX = dalloc<double>(cnt);
-        QK_HIP(hipMemcpyAsync(dX, hX, cnt * sizeof(double), hipMemcpyHostToDevice, s));
-        permute_block(s, dX, M, n, o, v);
+        RowUpload up(s, n1 * o, n2 * o * v);
+        up.rows(dX, ERI_MO + n1 * nC + n3 * nO, n1 * o, n1, n2, v, n3, 1, 0);
+        permute_block(s, dX, M, n, (int)o, (int)v);
         QK_HIP(hipStreamSynchronize(s));
     } catch (...) {
         (void)hipStreamSynchronize(s);
         dfree(dX);
-        (void)hipHostFree(hX);
         throw;
     }
     dfree(dX);
-    (void)hipHostFree(hX);
 }
 
 // upload rho(p,q,m) (QuAcK layout) into rhoT[m + nS (p + n q)]

@@ -212,6 +212,30 @@ struct AoScratch {
     double *t1 = nullptr, *t2 = nullptr;
 };
 AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf, size_t& cap, double* rhoT);
+// Rows of a host array to the device, one after the other.  The rows lie far apart in an
+// array that is in no cache (2.9 KB every 29 KB at N = 60), and a plain copy waits for each
+// row's first lines: 3.6 ms for the 9.3 MB of one block.  The lines of a row some 2 KB of
+// data ahead are asked for while a row is copied, and the copies leave from a short ring of
+// pinned slots while the next one fills (pinning a whole block costs 36 us a megabyte).
+struct RowUpload {
+    static constexpr int SLOTS = 3;
+    hipStream_t s;
+    size_t slot, turn = 0;  // doubles a slot; slots sent
+    double* h = nullptr;
+    hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr};
+    // for rows of up to `longest` values and calls of up to `total` values
+    RowUpload(hipStream_t s_, size_t longest, size_t total);
+    RowUpload(const RowUpload&) = delete;
+    RowUpload& operator=(const RowUpload&) = delete;
+    ~RowUpload() { release(); }
+    // n1 x n2 x n3 rows of len values at base + s1 i1 + s2 i2 + s3 i3, i1 fastest
+    void rows(double* dX, const double* base, size_t len, size_t n1, size_t s1, size_t n2, size_t s2, size_t n3,
+              size_t s3);
+
+  private:
+    void send(double* dst, size_t cnt);
+    void release();
+};
 void upload_mo_block(hipStream_t s, const double* ERI_MO, double* M, int n, int nC, int nO, int nR);
 // rho(p,q,m) (QuAcK layout, host) into rhoT[m + nS (p + n q)] on the device (caller frees)
 double* upload_rho(hipStream_t s, const double* rho, int n, int nS);

@@ -152,7 +152,7 @@ struct UScreen {
     const double* G[3];
     Ctx* c = nullptr;
     hipStream_t st = nullptr;
-    double* de = nullptr;
+    double *de = nullptr, *dX = nullptr;
     double *dM[2] = {nullptr, nullptr}, *dR[2] = {nullptr, nullptr};
     QpWork* q = nullptr;
 
@@ -190,23 +190,23 @@ struct UScreen {
             c->scal = dalloc<double>(8);
             c->info = dalloc<int>(1);
             de = dalloc<double>(2 * (size_t)n);
-            std::vector<double> Ms(n2 * nSt);
+            dX = dalloc<double>(n2 * std::max(nSa, nSb));
+            RowUpload host(st, (size_t)n * std::max(nO[0] - nC[0], nO[1] - nC[1]), n2 * std::max(nSa, nSb));
             for (int sp = 0; sp < 2; ++sp) {
                 dM[sp] = dalloc<double>(n2 * nSt);
                 dR[sp] = dalloc<double>(n2 * nSt);
-                for (int sj = 0; sj < 2; ++sj)
-                    for (int j = nC[sj]; j < nO[sj]; ++j)
-                        for (int b = 0; b < v[sj]; ++b) {
-                            const size_t k = (sj ? nSa : 0) + b + (size_t)v[sj] * (j - nC[sj]);
-                            const int Bb = nO[sj] + b;
-                            for (int qq = 0; qq < n; ++qq)
-                                for (int p = 0; p < n; ++p)
-                                    Ms[(p + (size_t)n * qq) + n2 * k] =
-                                        sp == 0 ? at(sj == 0 ? 0 : 1, p, j, qq, Bb)
-                                                : (sj == 0 ? at(1, j, p, Bb, qq) : at(2, p, j, qq, Bb));
-                        }
-                QK_HIP(hipMemcpyAsync(dM[sp], Ms.data(), sizeof(double) * n2 * nSt, hipMemcpyHostToDevice, st));
-                QK_HIP(hipStreamSynchronize(st));  // Ms is refilled for the next spin
+                for (int sj = 0; sj < 2; ++sj) {
+                    const size_t o = nO[sj] - nC[sj], b = v[sj], n3 = n2 * n;
+                    if (o * b == 0) continue;
+                    double* M = dM[sp] + (sj ? n2 * nSa : 0);  // M(p, q, b + v j) = (pq|jb), the spins sp and sj
+                    if (sp == 1 && sj == 0) {                  // G[1](j, p, b, q)
+                        host.rows(dX, G[1] + nC[0] + n2 * nO[0], o, n, n, b, n2, n, n3);
+                        permute_block_t(st, dX, M, n, (int)o, (int)b);
+                    } else {                                   // G[sp + sj](p, j, q, b)
+                        host.rows(dX, G[sp + sj] + (size_t)n * nC[sj] + n3 * nO[sj], n * o, n, n2, b, n3, 1, 0);
+                        permute_block(st, dX, M, n, (int)o, (int)b);
+                    }
+                }
             }
             extract_ku(st, dM[0], dM[1], c->K, up);
             const int rc = qk_gw_set_eigensolver(c, g_u_eig_mode.load(), g_u_eig_demax.load());
@@ -224,7 +224,7 @@ struct UScreen {
         if (st) (void)hipStreamSynchronize(st);
         delete q;
         q = nullptr;
-        for (double** p : {&de, &dM[0], &dM[1], &dR[0], &dR[1]}) dfree(*p);
+        for (double** p : {&de, &dX, &dM[0], &dM[1], &dR[0], &dR[1]}) dfree(*p);
         if (c) {
             std::copy(c->eig_count, c->eig_count + 9, g_u_eig_count);
             qk::release(c);
@@ -233,12 +233,9 @@ struct UScreen {
         }
         st = nullptr;
     }
-    double at(int k, int p, int qq, int r, int t) const {  // ERI_k(p, q, r, t), 0-based
-        return G[k][p + (size_t)n * (qq + (size_t)n * (r + (size_t)n * t))];
-    }
     // LR/phULR.f90 at energies en (n x 2, host); returns EcRPA, leaves Om and
-    // W = XpY^T on the device
-    double rpa(const double* en, const char* who) {
+    // W = XpY^T on the device (Om only without vectors)
+    double rpa(const double* en, const char* who, bool vectors = true) {
         if (!TDA_W) {
             // LR/phRLR.f90:57-58 (the unrestricted solver shares it): A - B
             // must be positive definite; here it is diag(e_a - e_i)
@@ -252,7 +249,7 @@ struct UScreen {
                          std::to_string(dmin) + "): linear-response instability");
         }
         QK_HIP(hipMemcpyAsync(de, en, sizeof(double) * 2 * n, hipMemcpyHostToDevice, st));
-        screening(c, de, en, TDA_W, true);
+        screening(c, de, en, TDA_W, vectors);
         double ec = 0.0;
         QK_HIP(hipMemcpyAsync(&ec, c->scal + 1, sizeof(double), hipMemcpyDeviceToHost, st));
         QK_HIP(hipStreamSynchronize(st));
@@ -364,8 +361,9 @@ int qk_ug0w0(int nBas, const int* nC, const int* nO, const int* nR, const double
             if (linearize) std::memcpy(eg, lin.data(), sizeof(double) * n);
             else u.qp(sp, doSRG, eta, es, lin.data(), es, eg, z);
         }
-        // RPA correlation energy at eGW (GW/UG0W0.f90:140-142)
-        const double ec = u.rpa(eGW, "qk_ug0w0 (RPA at eGW)");
+        // RPA correlation energy at eGW (GW/UG0W0.f90:140-142); a refining engine goes by
+        // its vectors, others need none
+        const double ec = u.rpa(eGW, "qk_ug0w0 (RPA at eGW)", u.c->eig_mode & 1);
         if (EcRPA) *EcRPA = ec;
     });
 }

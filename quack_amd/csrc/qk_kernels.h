@@ -37,6 +37,8 @@ struct UPairs {
 };
 
 void permute_block(hipStream_t s, const double* X, double* M, int n, int o, int v);
+// the same from X[j + o (p + n (b + v q))]
+void permute_block_t(hipStream_t s, const double* X, double* M, int n, int o, int v);
 // f (N^4, QuAcK's ERI.bin order) from the 8-fold packed chemists' array
 // (N(N+1)/2 pairs, pair-of-pairs packed)
 void unpack_eri_s8(hipStream_t s, const double* packed, double* f, int N);
