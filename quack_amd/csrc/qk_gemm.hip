@@ -174,8 +174,8 @@ void launch(hipStream_t s, int M, int N, int K, double alpha, const double* A, l
 }
 
 // Tile configurations: 0: 256 x 32, 1: 64 x 64, 2: 128 x 64, 3: 128 x 128;
-// 4: the library's rocblas_dgemm (only where lib_ok allows it).
-constexpr int NOWN = 4, CFG_LIB = 4, NCFG = 5;
+// 4: the library's rocblas_dgemm (only where lib_ok allows it); 5: 32 x 32 (not tuned).
+constexpr int NOWN = 4, CFG_LIB = 4, CFG_SMALL = 5, NCFG = 5;
 const char* const CFG_NAME[NCFG] = {"256x32", "64x64", "128x64", "128x128", "rocblas"};
 
 // Library FP64 GEMM as a tuning candidate (qk_set_library_gemm, off by
@@ -228,15 +228,22 @@ void launch_cfg(int cfg, hipStream_t s, int M, int N, int K, double alpha, const
         case 0: launch<4, 1, 4, 2, TA, TB>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt); break;
         case 1: launch<2, 2, 2, 2, TA, TB>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt); break;
         case 2: launch<2, 2, 4, 2, TA, TB>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt); break;
+        case CFG_SMALL: launch<2, 2, 1, 1, TA, TB>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt); break;
         default: launch<2, 2, 4, 4, TA, TB>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt); break;
     }
 }
 
-// fixed shape rule, used when tuning is off or not worth it
-int default_cfg(int M, int N) {
-    if (N <= 32) return 0;
-    if (N <= 64 || M <= 64) return 1;
-    return 3;
+// fixed shape rule, used when tuning is off or not worth it: the largest tile that still
+// gives every compute unit a workgroup, else the smallest.  One workgroup passes its slabs
+// one after the other, and a slab of a 128 x 128 tile is 64 matrix instructions a wave
+// (1.7 us with one wave a SIMD), of a 32 x 32 tile 4.  128 x 128 and now, us: 225^3 46 and
+// 14, 324^3 61 and 17, 474^3 83 and 24, 225 x 2812 x 225 48 and 21, 95^3 23 and 9.
+int default_cfg(int M, int N, int count) {
+    const auto tiles = [&](int b) { return (long long)((M + b - 1) / b) * ((N + b - 1) / b) * count; };
+    if (N <= 32 && tiles(32) >= 2048) return 0;
+    if (tiles(128) >= 256) return N <= 64 || M <= 64 ? 1 : 3;
+    if (tiles(64) >= 256) return 1;
+    return CFG_SMALL;
 }
 
 // Autotuner: the first call of a (TA, TB, M, N, K, batch, upper) shape with
@@ -264,7 +271,7 @@ int dispatch(hipStream_t s, int M, int N, int K, double alpha, const double* A, 
               long long ldb, double beta, double* C, long long ldc, const Batch& bt) {
     const double flop = 2.0 * M * N * (double)K * bt.count;
     if (!g_autotune.load() || beta != 0.0 || flop < 1e9) {
-        launch_cfg<TA, TB>(default_cfg(M, N), s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt);
+        launch_cfg<TA, TB>(default_cfg(M, N, bt.count), s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt);
         return 1;
     }
     const bool lib = lib_ok(s, M, N, K, lda, ldb, ldc, bt);
@@ -276,10 +283,10 @@ int dispatch(hipStream_t s, int M, int N, int K, double alpha, const double* A, 
         return 1;
     }
     if (stream_capturing(s)) {  // no timing inside a graph capture: an untuned shape keeps its default
-        launch_cfg<TA, TB>(default_cfg(M, N), s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt);
+        launch_cfg<TA, TB>(default_cfg(M, N, bt.count), s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bt);
         return 1;
     }
-    TuneEntry e{default_cfg(M, N), {0.f, 0.f, 0.f, 0.f, 0.f}};
+    TuneEntry e{default_cfg(M, N, bt.count), {0.f, 0.f, 0.f, 0.f, 0.f}};
     hipEvent_t ev[2] = {nullptr, nullptr};
     QK_HIP(hipEventCreate(&ev[0]));
     QK_HIP(hipEventCreate(&ev[1]));
