@@ -359,14 +359,20 @@ int qk_gwb_set_eri_ao_device(qk_gwb_handle h, const double* ERI_AO, long long st
     return guarded(&h->err, [&] {
         BStage st(h, 0);
         const bool sp = split_aotomo();
+        const Ctx* x0 = h->mol[0];
+        AoScratch w;
+        if (!sp)
+            w = ao_scratch(x0->nBas, x0->nOrb, x0->nC, x0->nO, x0->nR, x0->nS, h->aow, h->aow_doubles, h->rhoT,
+                           h->nmol);
         for (int m = 0; m < h->nmol; ++m) {
             Ctx* x = h->mol[m];
-            // one molecule after the other on the stream: they share the buffer
-            AoScratch w;
-            if (!sp)
-                w = ao_scratch(x->nBas, x->nOrb, x->nC, x->nO, x->nR, x->nS, h->aow, h->aow_doubles, x->rhoT);
-            aotomo_block(h->s, ERI_AO + m * stride_eri, c + m * stride_c, x->M, x->nBas, x->nOrb, x->nC, x->nO,
-                         x->nR, sp, x->K, w.t1, w.t2);
+            // groups one after the other on the stream: they share the buffers
+            if (w.group == 1)
+                aotomo_block(h->s, ERI_AO + m * stride_eri, c + m * stride_c, x->M, x->nBas, x->nOrb, x->nC, x->nO,
+                             x->nR, sp, x->K, w.t1, w.t2);
+            else if (m % w.group == 0)
+                aotomo_group(h->s, ERI_AO + m * stride_eri, stride_eri, c + m * stride_c, stride_c, x->M, x->nBas,
+                             x->nOrb, x->nC, x->nO, x->nR, std::min(w.group, h->nmol - m), w.t1, w.t2);
             if (!sp) extract_k(h->s, x->M, x->K, x->nOrb, x->nC, x->nO, x->v, x->nS);
             x->msplit_valid = false;
             x->have_eri = true;

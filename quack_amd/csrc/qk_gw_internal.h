@@ -207,11 +207,15 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
 bool split_aotomo();
 void aotomo_block(hipStream_t s, const double* f, const double* cc, double* M, int N, int n, int nC, int nO, int nR,
                   bool split = false, double* K = nullptr, double* work1 = nullptr, double* work2 = nullptr);
-// its two work arrays for a handle (null: it allocates); buf, cap: the handle's kept buffer
+void aotomo_group(hipStream_t s, const double* f, long long sF, const double* cc, long long sC, double* M, int N, int n,
+                  int nC, int nO, int nR, int cnt, double* work1, double* work2);
+// its two work arrays for a handle (null: it allocates), with room for `group` of nmol
+// molecules; buf, cap: the handle's kept buffer
 struct AoScratch {
     double *t1 = nullptr, *t2 = nullptr;
+    int group = 1;
 };
-AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf, size_t& cap, double* rhoT);
+AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf, size_t& cap, double* rhoT, int nmol);
 // Rows of a host array to the device, one after the other.  The rows lie far apart in an
 // array that is in no cache (2.9 KB every 29 KB at N = 60), and a plain copy waits for each
 // row's first lines: 3.6 ms for the 9.3 MB of one block.  The lines of a row some 2 KB of
