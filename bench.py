@@ -17,7 +17,7 @@ solution returns to that solution within 0.01 meV on every one of 40 seeded
 held-out H systems (eta = 0.05 with DIIS 5 does not on 6 of them), which is
 what makes the 1 meV comparisons meaningful.
 
-Forms: the plain FP64 form (QuAcK's arithmetic, dsyevd every cycle, one
+Forms: the plain FP64 form (QuAcK's arithmetic, full solve every cycle, one
 molecule at a time; median of --baseline-reps runs) is measured first as the
 accuracy reference and the baseline rate, then the same FP64 arithmetic with
 the project's own tridiagonalisation in every full solve; the timed form
@@ -312,8 +312,8 @@ def main():
                     help="fp64: QuAcK's arithmetic; mixed: excitation densities from three BF16 slices "
                          "(six products); mixed2: two slices (three products)")
     ap.add_argument("--eig", choices=["syevd", "refine", "sytrd", "refine+sytrd"], default="refine+sytrd",
-                    help="syevd: dsyevd every cycle (QuAcK); refine: Newton refinement of the previous eigenvectors, "
-                         "dsyevd for the rest; sytrd: full solves through the project's own tridiagonalisation; "
+                    help="syevd: full solve every cycle (QuAcK); refine: Newton refinement of the previous eigenvectors, "
+                         "full solves for the rest; sytrd: full solves through the project's own tridiagonalisation; "
                          "refine+sytrd: refinement, own-tridiagonalisation full solves for the rest")
     ap.add_argument("--de-max", type=float, default=0.03,
                     help="refinement is tried when no orbital energy moved by more than this (Ha) since the stored "
@@ -425,7 +425,7 @@ def run_h50(args):
             return wss[i].evgw(g, {"eHF": scf["eHF"], "Sx": scf["Sx"], "nO": nO})
         return g.evgw(scf["eHF"], **evkw)
 
-    # plain FP64 form (dsyevd every cycle, one molecule at a time): the accuracy
+    # plain FP64 form (full solve every cycle, one molecule at a time): the accuracy
     # reference of every molecule and, as the median of --baseline-reps runs on
     # the first molecule, the baseline rate
     for g in engs:
@@ -449,7 +449,7 @@ def run_h50(args):
     t = time.time()
     ref_own = step_on(0, False)
     t_fp64_own = time.time() - t
-    log("plain fp64 form, own tridiagonalisation: %.3f s/molecule, max |dE| vs dsyevd %.2e Ha" %
+    log("plain fp64 form, own tridiagonalisation: %.3f s/molecule, max |dE| vs mode 0 %.2e Ha" %
         (t_fp64_own, float(np.abs(ref_own["eGW"] - refs[0]["eGW"]).max())))
     st0 = eng.stage_times()  # the plain-form launches, part of the fp64 kernel's population only
 
@@ -602,7 +602,7 @@ def run_h50(args):
                    "step": "%d molecules" % K},
         "plain_fp64_form": {"molecules_per_s": 1.0 / t_fp64, "s_per_molecule_runs": t_fp64s,
                             "statistic": "median of %d runs, one molecule at a time" % len(t_fp64s),
-                            "cycles": refs[0].get("nSCF"), "eigensolver": "dsyevd every cycle",
+                            "cycles": refs[0].get("nSCF"), "eigensolver": "full solve every cycle",
                             "speedup_of_this_form": value * t_fp64},
         "plain_fp64_form_own_tridiagonal": {"molecules_per_s": 1.0 / t_fp64_own,
                                             "eigensolver": "own tridiagonalisation every cycle",

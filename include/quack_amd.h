@@ -141,11 +141,13 @@ int qk_gw_set_precision(qk_gw_handle h, int mode);
 
 /* Eigensolver of the RPA problem inside qk_evrgw, qk_gw_screen and the first
  * RPA of qk_rg0w0 (LR/phRLR.f90:77, diagonalize_matrix = dsyev):
- *   mode 0 (default): rocSOLVER dsyevd for every RPA, as QuAcK re-diagonalises
- *           every cycle;
- *   mode 2: full solves by the library's own Householder tridiagonalisation
- *           (LAPACK dsytrd layout), rocSOLVER dstedc on the tridiagonal and the
- *           library's own blocked back-transformation (in place of dormtr);
+ *   mode 0 (default): a full solve for every RPA, as QuAcK re-diagonalises
+ *           every cycle: the library's own kernels, or rocSOLVER dsyevd for
+ *           eigenvectors that go into split-precision densities;
+ *   mode 2: the same with the stages timed apart; eigenvectors for
+ *           split-precision densities by the library's own Householder
+ *           tridiagonalisation (LAPACK dsytrd layout), rocSOLVER dstedc on the
+ *           tridiagonal and the library's own blocked back-transformation;
  *   mode 1 (or 3 = 1 with the full solves of mode 2):
  *           when no orbital energy moved by more than de_max (Ha) since the
  *           handle's last eigenvectors were computed (same TDA_W), refine those
@@ -181,8 +183,8 @@ int qk_gw_qp_iters(qk_gw_handle h, int *nit);
  * [8], [9] the same two summed over every call since the handle was created;
  * [10] device time of the own Householder tridiagonalisations (eigensolver
  * modes 2 and 3) since the handle was created, [11] their number;
- * [12], [13] device time of the tridiagonal divide-and-conquer (rocSOLVER
- * dstedc) and of the own back-transformation in those solves with vectors.
+ * [12], [13] device time of the tridiagonal divide-and-conquer and of the own
+ * back-transformation in those solves with vectors.
  * n <= 14. */
 int qk_gw_stage_times(qk_gw_handle h, double *ms, int n);
 
@@ -291,11 +293,11 @@ int qk_ugw_phbse(int nBas, const int *nC, const int *nO, const int *nR, const do
                  int spin_conserved, int spin_flip, int exchange_kernel, double *EcBSE, double *OmSC, double *OmSF);
 
 /* Eigensolver of the unrestricted screening of qk_ug0w0 and qk_evugw,
- * process-wide: mode and de_max as qk_gw_set_eigensolver (0: rocSOLVER dsyevd
- * for every RPA, QuAcK's sequence and the default; 1: Newton refinement of the
+ * process-wide: mode and de_max as qk_gw_set_eigensolver (0: a full solve for
+ * every RPA, QuAcK's sequence and the default; 1: Newton refinement of the
  * previous cycle's eigenvectors when no energy of either spin moved by more
- * than de_max Ha, dsyevd otherwise; 2: the own tridiagonalisation for every
- * full solve; 3: both).  No counterpart in QuAcK (LR/phULR.f90 always calls
+ * than de_max Ha, a full solve otherwise; 2, 3: as 0, 1 with the stages timed
+ * apart).  No counterpart in QuAcK (LR/phULR.f90 always calls
  * diagonalize_matrix). */
 int qk_set_unrestricted_eigensolver(int mode, double de_max);
 /* Eigensolver counts (as qk_gw_eig_stats) of the calling thread's last

@@ -17,6 +17,9 @@
 // a small kernel prepares the first column of each panel, and after each
 // panel the trailing update A -= V W^T + W V^T runs as two matrix-core GEMMs
 // on the upper tiles.  No host synchronisation inside.
+// This launched form serves eigenvectors of split-precision contractions (their bits are
+// kept), orders above 3072 and a register-resident launch (qk_trdres.hip) that gave up;
+// eigh() below puts the FP64 full solve together.
 #include <algorithm>
 
 #include "qk_kernels.h"

@@ -226,10 +226,12 @@ class GWEngine:
         _check(load().qk_gw_set_precision(self.h, PRECISION.get(mode, mode)), self.h)
 
     def set_eigensolver(self, mode, de_max=5e-3):
-        """"syevd" (0): dsyevd for every RPA, QuAcK's scheme; "refine" (1):
-        Newton refinement of the previous eigenvectors when no orbital energy
-        moved by more than de_max Ha, dsyevd otherwise; "sytrd" (2): full solves
-        through the library's own tridiagonalisation; "refine+sytrd" (3)."""
+        """"syevd" (0): a full solve for every RPA, QuAcK's scheme (rocSOLVER's
+        dsyevd where the eigenvectors go into split-precision densities, the
+        library's own kernels otherwise); "refine" (1): Newton refinement of the
+        previous eigenvectors when no orbital energy moved by more than de_max
+        Ha, a full solve otherwise; "sytrd" (2), "refine+sytrd" (3): the same
+        with the library's own tridiagonalisation in every full solve."""
         _check(load().qk_gw_set_eigensolver(self.h, EIG_MODES.get(mode, mode), de_max), self.h)
 
     def eig_stats(self):
