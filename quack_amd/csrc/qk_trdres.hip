@@ -21,8 +21,12 @@
 // words, half of the value beside the column number, stored and loaded with
 // single agent-scope atomics, so a reader that sees the column number has the
 // value (one trip through the shared cache instead of store, counter, poll and
-// load).  Two buffers alternate: a workgroup can write column c-2 only after
-// it has read every workgroup's column c-1, which they publish after reading c.
+// load).  Two buffers alternate, so a reader of column c has to be done before anyone
+// writes column c-2.  A writer of c-2 has read the y of column c-1 of every workgroup that
+// has a row there (g < c-1), and those publish it after reading c.  The others must not
+// read c: workgroup g > 0 leaves once it has published column g+1, its last rows' y, and
+// the reflector goes to memory from the workgroup of row c-1, which has one in column c.
+// (Workgroup 0 has row 0 in every column and stays to the end.)
 //
 // Two shapes of the same algorithm: k_trd_small (n <= 160) is one workgroup and
 // needs no exchange; k_trd_wide (n <= 3072) spreads the columns over the 512
@@ -350,7 +354,8 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
     if (tid == 0) quit = 0;
     lds_barrier();
     unsigned spins = 0;
-    for (; c >= 1; --c) {
+    const int last = g == 0 ? 1 : g + 1;  // the last column this workgroup has a row in
+    for (; c >= last; --c) {
         const int par = c & 1;
         // row c-1, brought up to date, goes to everyone first: it is on its way while the
         // reflector and y are worked out
@@ -402,7 +407,7 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
                 publish(X + 4LL * n * par + 2 * r, tree_sum<NT / 64>(&yp[0][tid], R), c);
             }
         }
-        if (V && g == c % G) {
+        if (V && g == (c - 1) % G) {
 #pragma unroll
             for (int k = 0; k < KC; ++k) {
                 const int col = tid + NT * k;
@@ -413,6 +418,7 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
             E[c - 1] = h.beta;
             TAU[c - 1] = h.tau;
         }
+        if (g > 0 && c == last) return;
         double y[KC], dot = 0.0;
         {
             long long t0 = 0;
