@@ -33,7 +33,8 @@ enum {
     QK_OK = 0,
     QK_E_ARG = 1,          /* invalid size, flag or pointer */
     QK_E_HIP = 2,          /* HIP runtime or device error */
-    QK_E_EIG = 3,          /* eigensolver failure (rocSOLVER info != 0) */
+    QK_E_EIG = 3,          /* eigensolver failure: a matrix that is not finite
+                            * (levels that cross, a NaN integral), rocSOLVER info != 0 */
     QK_E_NOCONV = 4,       /* evGW reached maxSCF+1 cycles (GW/evRGW.f90:190-199) */
     QK_E_UNSUPPORTED = 5,  /* option not implemented on the GPU path */
     QK_E_ALLOC = 6,        /* device memory exhausted */

@@ -61,8 +61,10 @@ __device__ inline double rsq2(double x) {
 
 // ---- scaling, bounds ----------------------------------------------------------
 // One block per matrix: a power-of-two scale that brings max |T| to [1/2, 1), the
-// Gershgorin interval, and info = 1 where an entry is not finite.
-// hd: [0] scale, [1] 1/scale, [2] lower bound, [3] upper bound;
+// Gershgorin interval, and info = 1 where an entry is not finite.  Such a matrix goes
+// on as zeros (k_dc_leaf, k_dc_setup) and its values come out as NaN: the merges below
+// index by the order of their values, which must be numbers.
+// hd: [0] scale, [1] 1/scale, [2] lower bound, [3] upper bound, [4] 1 where not finite;
 // de: 2 n scaled pairs (d_i, e_{i-1}^2) for the counts (null: not wanted).
 __global__ __launch_bounds__(256) void k_tri_prep(const double* __restrict__ D, const double* __restrict__ E,
                                                   long long sd, int n, double* __restrict__ hd, double* __restrict__ de,
@@ -113,6 +115,7 @@ __global__ __launch_bounds__(256) void k_tri_prep(const double* __restrict__ D, 
         hd[1] = ldexp(1.0, ex);
         hd[2] = lo - m;
         hd[3] = hi + m;
+        hd[4] = anybad ? 1.0 : 0.0;
         info[z] = anybad ? 1 : 0;
     }
 }
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(256) void k_tri_values(const double* __restrict__ d
         lo = f > 0 ? xl : lo;
         hi = f < LPE ? xh : hi;
     }
-    if (l == 0 && g < n) w[z * sw + g] = 0.5 * (lo + hi) * back;
+    if (l == 0 && g < n) w[z * sw + g] = hd[8LL * z + 4] == 0.0 ? 0.5 * (lo + hi) * back : __builtin_nan("");
 }
 
 // ---- leaves --------------------------------------------------------------------------
@@ -202,6 +205,7 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
     D += z * sd;
     E += z * sd;
     const double scale = hd[8LL * z];
+    const bool ok = hd[8LL * z + 4] == 0.0;
     const int p0 = cut(n, blockIdx.x, k), p1 = cut(n, blockIdx.x + 1, k), m = p1 - p0;
     for (int x = t; x < LEAF * LD; x += 64) {
         A[x] = 0.0;
@@ -212,9 +216,9 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
         double v = D[p0 + t] * scale;
         if (t == 0 && p0 > 0) v -= fabs(E[p0 - 1]) * scale;
         if (t == m - 1 && p1 < n) v -= fabs(E[p1 - 1]) * scale;
-        A[t * LD + t] = v;
+        A[t * LD + t] = ok ? v : 0.0;
         V[t * LD + t] = 1.0;
-        if (t + 1 < m) A[t * LD + t + 1] = A[(t + 1) * LD + t] = E[p0 + t] * scale;
+        if (t + 1 < m) A[t * LD + t + 1] = A[(t + 1) * LD + t] = ok ? E[p0 + t] * scale : 0.0;
     }
     __syncthreads();
     const int me = (m + 1) & ~1;  // players (one may sit out)
@@ -282,7 +286,7 @@ __global__ __launch_bounds__(64) void k_dc_leaf(const double* __restrict__ D, co
         const int r = x % m, c = x / m;
         int rank = 0;
         for (int i = 0; i < m; ++i) rank += dv[i] < dv[c] || (dv[i] == dv[c] && i < c);
-        rank = min(rank, m - 1);  // (values that are not numbers)
+        rank = min(rank, m - 1);
         Q[(p0 + r) + (long long)n * (p0 + rank)] = V[r * LD + c];
         if (r == 0) d[z * sdd + p0 + rank] = dv[c];
     }
@@ -347,12 +351,17 @@ __global__ __launch_bounds__(ST) void k_dc_setup(Dc a) {
     const long long o = z * a.sm + s;
     const double* d = a.d + o;
     const double scale = a.hd[8LL * z];
-    const double e = a.E[z * a.sE + m - 1] * scale;
+    const double e = a.hd[8LL * z + 4] == 0.0 ? a.E[z * a.sE + m - 1] * scale : 0.0;
     const double rho = 2.0 * fabs(e), sg = (e < 0.0 ? -1.0 : 1.0) * 0.70710678118654752440;
     const double* Q = a.Q + z * a.sQ + (long long)a.n * s;
     // sorted merge of the halves into mu (values), lam (z), org (columns): free until the roots
     double *ds = a.mu + o, *zs = a.lam + o;
     int* src = a.org + o;
+    // The places p are a permutation because each half's values ascend: k_dc_leaf sorts
+    // them, and later ones are roots between poles that lie more than tol apart, and
+    // deflated values by rank.  (Columns read back from src are held inside the node all
+    // the same: a wrong one would send k_dc_gemm out of Q.)
+    const auto source = [&](int i) { return (int)min((unsigned)src[i], (unsigned)(N - 1)); };
     double md = 0.0, mz = 0.0;
     for (int i = tid; i < N; i += ST) {
         const double x = d[i];
@@ -400,13 +409,13 @@ __global__ __launch_bounds__(ST) void k_dc_setup(Dc a) {
         if (keep) {
             cd[M + r] = x;
             cz[M + r] = zz;
-            csrc[M + r] = src[i];
-            cty[M + r] = src[i] < n1 ? 0 : 2;
+            csrc[M + r] = source(i);
+            cty[M + r] = source(i) < n1 ? 0 : 2;
             cfl[M + r] = 1;
         } else if (i < N) {
             const int q = nd + tid - r;  // dropped so far
             dd[q] = x;
-            dcol[q] = src[i];
+            dcol[q] = source(i);
         }
         M += tot;
         nd += min(ST, N - b) - tot;
@@ -794,11 +803,11 @@ __global__ __launch_bounds__(256, 2) void k_dc_gemm(Dc a, int tm, int tn) {
     }
 }
 
-// w = d / scale
+// w = d / scale (NaN for a matrix that is not finite)
 __global__ void k_dc_out(const double* __restrict__ d, long long sdd, const double* __restrict__ hd, int n,
                          double* __restrict__ w, long long sw) {
     const int i = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y;
-    if (i < n) w[z * sw + i] = d[z * sdd + i] * hd[8LL * z + 1];
+    if (i < n) w[z * sw + i] = hd[8LL * z + 4] == 0.0 ? d[z * sdd + i] * hd[8LL * z + 1] : __builtin_nan("");
 }
 
 __global__ void k_dc_zero(double* __restrict__ x, long long count) {
