@@ -926,21 +926,25 @@ AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf,
 
 // LR/phRLR.f90 for a number of problems of one order side by side on the device: the
 // caller fills A and B (S2 apart), solve() leaves Om in w, EcRPA in sc[4 m + 1] and,
-// with vectors, X + Y in ApB and X - Y in B (A and B under TDA: X in B).
+// with vectors, X + Y in xpy() and X - Y in xmy().
 // Both eigensolves are one launch chain for all problems, and those that nobody asks
 // eigenvectors of are values only: singlet and triplet BSE of N = 60 (nS = 324) cost two
 // tridiagonalisations, 1.5 ms, where one spin after the other took four, 3.0 ms.
+// QuAcK's diagonalize_matrix reads the upper triangles of A - B and of
+// Z = (A - B)^1/2 (A + B) (A - B)^1/2.  Where A and B are symmetric any basis does for Z,
+// and that of A - B saves two products; Z of others is formed in the pairs' own basis,
+// whose upper triangle it is.
 struct PhRlr {
     hipStream_t s;
     int nS, batch, tda;
-    bool vectors;
+    bool vectors, symmetric;
     size_t S2;
     double *A = nullptr, *B = nullptr, *U = nullptr, *ApB = nullptr, *T = nullptr, *Ti = nullptr;
     double *w = nullptr, *work = nullptr, *sc = nullptr;
     int* info = nullptr;
     Error err{QK_OK, ""};  // of the first problem that failed
-    PhRlr(hipStream_t s_, int nS_, int batch_, int tda_, bool vec)
-        : s(s_), nS(nS_), batch(batch_), tda(tda_), vectors(vec), S2((size_t)nS_ * nS_) {
+    PhRlr(hipStream_t s_, int nS_, int batch_, int tda_, bool vec, bool sym)
+        : s(s_), nS(nS_), batch(batch_), tda(tda_), vectors(vec), symmetric(sym), S2((size_t)nS_ * nS_) {
         try {
             A = dalloc<double>(S2 * batch);
             U = dalloc<double>(S2 * batch);
@@ -1009,8 +1013,8 @@ struct PhRlr {
             if (nb > 0) rpa_finalize(s, w, nullptr, nullptr, sc, nS, 1, false, zs, nb);
             return nb;
         }
-        // LR/phRLR.f90:47-81 with A - B = U d U^T in its eigenvectors' basis:
-        // T = U d^1/2, Z = T^T (A + B) T, (X + Y)^T = T V Om^-1/2, (X - Y)^T = U d^-1/2 V Om^1/2
+        // LR/phRLR.f90:47-81 with A - B = U d U^T, T = U d^1/2 and, in its eigenvectors' basis,
+        // Z = T^T (A + B) T, (X + Y)^T = T V Om^-1/2, (X - Y)^T = U d^-1/2 V Om^1/2
         apb_amb(s, A, B, ApB, U, (long long)(S2 * nb));
         nb = eig(nb, true, true);
         if (nb == 0) return 0;
@@ -1021,24 +1025,37 @@ struct PhRlr {
         Batch b;
         b.zdiv = b.count = nb;
         b.sa0 = b.sb0 = b.sc0 = (long long)S2;
-        dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, T, nS, 0.0, A, nS, b);
-        dgemm(s, true, false, nS, nS, nS, 1.0, T, nS, A, nS, 0.0, U, nS, b);
+        if (symmetric) {
+            dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, T, nS, 0.0, A, nS, b);
+            dgemm(s, true, false, nS, nS, nS, 1.0, T, nS, A, nS, 0.0, U, nS, b);
+        } else {
+            // B = (A - B)^1/2, A = (A - B)^-1/2
+            dgemm(s, false, true, nS, nS, nS, 1.0, T, nS, U, nS, 0.0, B, nS, b);
+            if (vectors) dgemm(s, false, true, nS, nS, nS, 1.0, Ti, nS, U, nS, 0.0, A, nS, b);
+            dgemm(s, false, false, nS, nS, nS, 1.0, ApB, nS, B, nS, 0.0, T, nS, b);
+            dgemm(s, false, false, nS, nS, nS, 1.0, B, nS, T, nS, 0.0, U, nS, b);
+        }
         nb = eig(nb, vectors, false);
         if (nb == 0) return 0;
         b.zdiv = b.count = nb;
         rpa_finalize(s, w, nullptr, nullptr, sc, nS, 0, false, zs, nb);  // Om = sqrt|w|
         if (vectors) {
-            dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, T, nS, 0.0, ApB, nS, b);
-            dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, Ti, nS, 0.0, B, nS, b);
+            if (symmetric) {
+                dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, T, nS, 0.0, ApB, nS, b);
+                dgemm(s, true, true, nS, nS, nS, 1.0, U, nS, Ti, nS, 0.0, B, nS, b);
+            } else {
+                dgemm(s, true, false, nS, nS, nS, 1.0, U, nS, B, nS, 0.0, ApB, nS, b);
+                dgemm(s, true, false, nS, nS, nS, 1.0, U, nS, A, nS, 0.0, T, nS, b);
+            }
             for (int m = 0; m < nb; ++m) {
                 rowscale_pow(s, ApB + S2 * m, w + (size_t)nS * m, nS, -0.5);
-                rowscale_pow(s, B + S2 * m, w + (size_t)nS * m, nS, 0.5);
+                rowscale_pow(s, (symmetric ? B : T) + S2 * m, w + (size_t)nS * m, nS, 0.5);
             }
         }
         return nb;
     }
     const double* xpy() const { return tda ? B : ApB; }
-    const double* xmy() const { return B; }
+    const double* xmy() const { return tda || symmetric ? B : T; }
 };
 
 // The four-index block M is allocated on first use (a density-fitted handle never needs it).
@@ -1727,7 +1744,7 @@ int qk_phrlr(int TDA, int nS, const double* Aph, const double* Bph, double* EcRP
     if (nS <= 0 || !Aph || (!TDA && !Bph) || !Om || !XpY || !XmY) return QK_E_ARG;
     return guarded(nullptr, [&] {
         hipStream_t s = scratch().s;
-        PhRlr r(s, nS, 1, TDA, true);
+        PhRlr r(s, nS, 1, TDA, true, false);
         QK_HIP(hipMemcpyAsync(r.A, Aph, sizeof(double) * r.S2, hipMemcpyHostToDevice, s));
         if (!TDA) QK_HIP(hipMemcpyAsync(r.B, Bph, sizeof(double) * r.S2, hipMemcpyHostToDevice, s));
         if (r.solve() != 1) throw r.err;
@@ -1898,7 +1915,7 @@ int qk_rgw_phbse_dyn(int dophBSE2, int exchange_kernel, int TDA_W, int TDA, int 
         std::unique_ptr<PhRlr> lr;
         int solved = 0;
         if (nspin > 0) {
-            lr.reset(new PhRlr(c->s, nS, nspin, TDA, dBSE != 0));
+            lr.reset(new PhRlr(c->s, nS, nspin, TDA, dBSE != 0, true));
             // the integrals of A and B: D1(b,i,j,a) = ERI(b,i,j,a), D2(b,j,a,i) = ERI(b,j,a,i)
             std::vector<double> hD(2 * S2);
             double *D1 = hD.data(), *D2 = D1 + S2;
