@@ -169,6 +169,15 @@ int qk_gw_set_eigensolver(qk_gw_handle h, int mode, double de_max);
  * cluster met; full solves by the own tridiagonalisation. */
 int qk_gw_eig_stats(qk_gw_handle h, long long *counts, int n);
 
+/* The full solves of a handle keep a matrix of order 161 to 3072 in the registers
+ * of workgroups that wait for each other inside one launch.  Where another
+ * process holds a part of the same GPU such a wait can fail; it ends after 2 s, and
+ * this and the handle's later solves use one launch per column and step instead (the
+ * same energies to rounding).  mode 1: this GPU is shared, use those at once; 0: start
+ * with the registers again (the default); 2: as 0, and count the next launch as
+ * one that failed, to try what follows it.  No counterpart in QuAcK. */
+int qk_gw_set_shared_device(qk_gw_handle h, int mode);
+
 /* Newton iterations of every orbital in the handle's last graphical QP solve
  * (nit[nOrb]; 64 = QuAcK's maxIt, where the orbital keeps its starting energy,
  * GW/RGW_QP_graph.f90:78-81; 0 for frozen orbitals).  No counterpart in QuAcK,
@@ -420,6 +429,8 @@ int qk_gwb_stage_times(qk_gwb_handle h, double *ms, int n);
  * eigensolver's info after each cycle.  Results are identical with it on or
  * off.  No counterpart in QuAcK (GW/evRGW.f90:119-183 is the cycle). */
 int qk_gwb_set_graphs(qk_gwb_handle h, int on);
+/* qk_gw_set_shared_device for a batch. */
+int qk_gwb_set_shared_device(qk_gwb_handle h, int mode);
 /* counts[0] = evGW cycles run eagerly, counts[1] = cycles replayed from graphs
  * (since the handle was created), n <= 2 */
 int qk_gwb_graph_stats(qk_gwb_handle h, long long *counts, int n);

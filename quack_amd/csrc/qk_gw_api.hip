@@ -29,8 +29,9 @@ void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double
 
 const char* const NOT_FINITE = "eigensolver: the matrix has entries that are not finite";
 
-void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, hipEvent_t* tev) {
-    eigh(s, n, 1, A, (long long)n * n, w, n, vectors, work, dinfo, tev);
+void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, Resident& resident,
+                  hipEvent_t* tev) {
+    eigh(s, n, 1, A, (long long)n * n, w, n, vectors, work, dinfo, resident, tev);
     int info = 0;
     QK_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
     QK_HIP(hipStreamSynchronize(s));
@@ -146,7 +147,7 @@ void syevd_own(hipStream_t s, rocblas_handle rb, int n, double*& A, double* w, d
                double* work, double* owork, int* dinfo, hipEvent_t* tev, SolveGraphs* gr) {
     QK_HIP(hipEventRecord(tev[0], s));
     double* Ain = A;
-    run_graph(s, gr->trd, Ain, [&] { sytrd_upper(s, n, Ain, w, E, tau, work, 32, nullptr, false); });
+    run_graph(s, gr->trd, Ain, [&] { sytrd_upper(s, n, Ain, w, E, tau, work, 32, nullptr, nullptr); });
     QK_HIP(hipEventRecord(tev[1], s));
     rb_check(rocsolver_dstedc(rb, rocblas_evect_tridiagonal, n, w, E, Z, n, dinfo), "rocsolver_dstedc");
     QK_HIP(hipEventRecord(tev[2], s));
@@ -555,7 +556,7 @@ void solve_full(Ctx* c, bool vectors) {
         c->eigw = dalloc<double>(need);
         c->eigw_doubles = need;
     }
-    eigh_checked(c->s, c->nS, c->Cm, c->Om, vectors, c->eigw, c->info, c->eig_mode & 2 ? c->ev3 : nullptr);
+    eigh_checked(c->s, c->nS, c->Cm, c->Om, vectors, c->eigw, c->info, c->resident, c->eig_mode & 2 ? c->ev3 : nullptr);
 }
 
 // The same for eigenvectors of a split-precision contraction, modes 2 and 3.
@@ -942,6 +943,7 @@ struct PhRlr {
     double *A = nullptr, *B = nullptr, *U = nullptr, *ApB = nullptr, *T = nullptr, *Ti = nullptr;
     double *w = nullptr, *work = nullptr, *sc = nullptr;
     int* info = nullptr;
+    Resident resident;
     Error err{QK_OK, ""};  // of the first problem that failed
     PhRlr(hipStream_t s_, int nS_, int batch_, int tda_, bool vec, bool sym)
         : s(s_), nS(nS_), batch(batch_), tda(tda_), vectors(vec), symmetric(sym), S2((size_t)nS_ * nS_) {
@@ -973,7 +975,7 @@ struct PhRlr {
     }
     // the eigensolve of the first nb matrices in U; returns how many of them stand
     int eig(int nb, bool vec, bool positive) {
-        eigh(s, nS, nb, U, (long long)S2, w, nS, vec, work, info);
+        eigh(s, nS, nb, U, (long long)S2, w, nS, vec, work, info, resident);
         std::vector<int> bad(nb);
         std::vector<double> low(nb);
         QK_HIP(hipMemcpyAsync(bad.data(), info, sizeof(int) * nb, hipMemcpyDeviceToHost, s));
@@ -1508,6 +1510,12 @@ int qk_gw_set_precision(qk_gw_handle c, int mode) {
     return guarded(&c->err, [&] {
         c->precision = mode;  // slices are allocated on first use
     });
+}
+
+int qk_gw_set_shared_device(qk_gw_handle c, int mode) {
+    if (!c || mode < 0 || mode > 2) return QK_E_ARG;
+    c->resident = Resident{mode == 1, mode == 2};
+    return QK_OK;
 }
 
 int qk_gw_set_eigensolver(qk_gw_handle c, int mode, double de_max) {

@@ -21,6 +21,7 @@ struct qk_gwb_ctx {
     int *info = nullptr, *active = nullptr, *nit = nullptr, *done = nullptr;
     double* eigw = nullptr;  // work of the eigensolves, on first use
     size_t eigw_doubles = 0;
+    qk::Resident resident;
     double* aow = nullptr;  // work of aotomo_block, on first use
     size_t aow_doubles = 0;
     qk::Zs zs;
@@ -96,7 +97,7 @@ void solve_batch(BCtx* b, bool vectors, bool check) {
             b->eigw = dalloc<double>(need);
             b->eigw_doubles = need;
         }
-        eigh(b->s, nS, b->nmol, b->Cm, S2, b->Om, nS, vectors, b->eigw, b->info);
+        eigh(b->s, nS, b->nmol, b->Cm, S2, b->Om, nS, vectors, b->eigw, b->info, b->resident);
     }
     if (check) {
         std::vector<int> info(b->nmol);
@@ -334,6 +335,12 @@ int qk_gwb_set_precision(qk_gwb_handle h, int mode) {
     if (!h || mode < 0 || mode > 2) return QK_E_ARG;
     h->precision = mode;
     for (Ctx* c : h->mol) c->precision = mode;
+    return QK_OK;
+}
+
+int qk_gwb_set_shared_device(qk_gwb_handle h, int mode) {
+    if (!h || mode < 0 || mode > 2) return QK_E_ARG;
+    h->resident = Resident{mode == 1, mode == 2};
     return QK_OK;
 }
 

@@ -61,7 +61,7 @@ inline rocblas_handle blas(rocblas_handle& rb, hipStream_t s) {
 // rocSOLVER dsyevd with eigenvectors on the stream bound to rb; eigenvalues ascending in w
 void syevd(hipStream_t s, rocblas_handle rb, int n, double* A, double* w, double* work, int* dinfo);
 // eigh of one n x n matrix, waited for; QK_E_EIG when it has entries that are not finite
-void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo,
+void eigh_checked(hipStream_t s, int n, double* A, double* w, bool vectors, double* work, int* dinfo, Resident& resident,
                   hipEvent_t* tev = nullptr);
 
 struct GraphSlot {
@@ -156,6 +156,7 @@ struct qk_gw_ctx {
     bool keep_syevd = false;  // qsGW's engine: eigenvectors from rocSOLVER dsyevd
     double* eigw = nullptr;   // work of the full solves, on first use
     size_t eigw_doubles = 0;
+    qk::Resident resident;
     double* aow = nullptr;  // work of aotomo_block, on first use
     size_t aow_doubles = 0;
     double *Zev = nullptr, *tau = nullptr, *trd_work = nullptr, *orm_work = nullptr;  // split-precision full solves

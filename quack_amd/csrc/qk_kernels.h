@@ -139,14 +139,28 @@ void mix_rows(hipStream_t s, double* A, int n, const int* idx, const int* ptr, c
 void gather_cols(hipStream_t s, const double* X, int n, const int* idx, int m, double* out);
 // (i, a) block of density-fitting factors: Bov[P + naux ia] = B[P + naux (i + n a)]
 void gather_bov(hipStream_t s, const double* B, double* Bov, int naux, int n, int nC, int nO, int v, int nS);
+// Whether an owner's solves use the launches whose workgroups wait for each other
+// (qk_trdres.hip).  A launch that gave a wait up, because another process holds a part of
+// the device, cost 2 s; the owner's later solves take the launched form at once.
+struct Resident {
+    bool off = false;
+    bool rehearse = false;  // the next such launch counts as given up
+    // after such a launch, with its flag read
+    bool gave_up(int fail) {
+        off = off || fail || rehearse;
+        rehearse = false;
+        return off;
+    }
+};
+
 // Householder tridiagonalisation, upper triangle, LAPACK dsytrd layout (qk_sytrd.hip);
 // work holds sytrd_work_doubles(n, nb) doubles, nb <= 64.
 size_t sytrd_work_doubles(int n, int nb);
-// With resident, the last columns run in registers (qk_trdres.hip): no graph capture,
-// and one host wait.  Returns the order m of that part (0: none): its reflectors
-// are in V only (or nowhere, if null), the others in A only.
+// With resident, and where that allows it, the last columns run in registers
+// (qk_trdres.hip): no graph capture, and one host wait.  Returns the order m of that
+// part (0: none): its reflectors are in V only (or nowhere, if null), the others in A only.
 int sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, double* V,
-                bool resident);
+                Resident* resident);
 // Z <- Q Z with the reflectors sytrd_upper (not resident) left in A, TAU (LAPACK
 // dormtr, SIDE = 'L', UPLO = 'U', TRANS = 'N'); work holds ormtr_work_doubles(n).
 size_t ormtr_work_doubles(int n);
@@ -164,6 +178,7 @@ void permute_cols(hipStream_t s, const double* X, const int* perm, double* out, 
 // has to be read, and the outputs are void where it is set.
 int trd_resident_max();
 bool trd_resident_fits(int n);
+bool trd_resident_waits(int n, int batch);  // whether trd_resident() will return true
 size_t trd_resident_words(int n, int batch);
 const int* trd_resident_fail(int n, int batch, const double* words);
 bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
@@ -198,6 +213,6 @@ void orm_strip_apply(hipStream_t s, int n, int batch, double* Z, long long sZ, d
 // back-transformation (the last two with vectors only).
 size_t eigh_work_doubles(int n, int batch, bool vectors);
 void eigh(hipStream_t s, int n, int batch, double* A, long long sA, double* w, long long sw, bool vectors, double* work,
-          int* info, hipEvent_t* tev = nullptr);
+          int* info, Resident& resident, hipEvent_t* tev = nullptr);
 
 }  // namespace qk

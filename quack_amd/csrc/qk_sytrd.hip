@@ -627,20 +627,19 @@ void sytrd_columns(hipStream_t s, int n, double* A, double* D, double* E, double
 }  // namespace
 
 int sytrd_upper(hipStream_t s, int n, double* A, double* D, double* E, double* TAU, double* work, int nb, double* V,
-                bool resident) {
+                Resident* resident) {
     QK_CHECK(n >= 1 && nb >= 1 && nb <= 64, QK_E_ARG, "sytrd: bad size");
     // 0-based columns n-1 down to 1 carry reflectors.  Those of the leading block
     // that fits the registers run there: at n = 1326 4.8 ms instead of 22.
     const int m = std::min(n, trd_resident_max());
-    if (resident && trd_resident_fits(m)) {
+    if (resident && !resident->off && trd_resident_fits(m)) {
         sytrd_columns(s, n, A, D, E, TAU, work, nb, n - 1, m);
         double* words = work + sytrd_work_doubles(n, nb) - trd_resident_words(m, 1);
+        if (!trd_resident(s, m, A, n, 0, V, n, 0, D, E, TAU, 0, 1, words)) return m;
         int fail = 0;
-        if (trd_resident(s, m, A, n, 0, V, n, 0, D, E, TAU, 0, 1, words)) {
-            QK_HIP(hipMemcpyAsync(&fail, trd_resident_fail(m, 1, words), sizeof(int), hipMemcpyDeviceToHost, s));
-            QK_HIP(hipStreamSynchronize(s));
-        }
-        if (!fail) return m;
+        QK_HIP(hipMemcpyAsync(&fail, trd_resident_fail(m, 1, words), sizeof(int), hipMemcpyDeviceToHost, s));
+        QK_HIP(hipStreamSynchronize(s));
+        if (!resident->gave_up(fail)) return m;
         // another process's launch shares the device: A still holds the block
         sytrd_columns(s, n, A, D, E, TAU, work, nb, m - 1, 1);
     } else {
@@ -782,7 +781,7 @@ struct EighWork {
 size_t eigh_work_doubles(int n, int batch, bool vectors) { return EighWork(n, batch, vectors, nullptr).total; }
 
 void eigh(hipStream_t s, int n, int batch, double* A, long long sA, double* w, long long sw, bool vectors, double* work,
-          int* info, hipEvent_t* tev) {
+          int* info, Resident& resident, hipEvent_t* tev) {
     QK_CHECK(n >= 1 && batch >= 1, QK_E_ARG, "eigh: bad size");
     const EighWork k(n, batch, vectors, work);
     // the columns of Z fit the registers up to order 2048; larger ones go through GEMMs
@@ -797,20 +796,22 @@ void eigh(hipStream_t s, int n, int batch, double* A, long long sA, double* w, l
         else ormtr_prepare(s, n, count, Az, sA, tz, n, wz, sW, m);
     };
     if (tev) QK_HIP(hipEventRecord(tev[0], s));
-    int fail = 0;
-    const bool whole = trd_resident_fits(n);
+    // (one workgroup a matrix waits for nobody, whatever holds the device)
+    bool whole = trd_resident_fits(n) && !(resident.off && trd_resident_waits(n, batch));
     if (whole && trd_resident(s, n, A, n, sA, k.orm, ldv, sW, k.D, k.E, k.TAU, n, batch, k.words)) {
+        int fail = 0;
         QK_HIP(hipMemcpyAsync(&fail, trd_resident_fail(n, batch, k.words), sizeof(int), hipMemcpyDeviceToHost, s));
         QK_HIP(hipStreamSynchronize(s));
+        whole = !resident.gave_up(fail);
     }
-    if (whole && !fail) {
+    if (whole) {
         if (tev) QK_HIP(hipEventRecord(tev[1], s));
         prepare(0, batch, n);
     } else {
         for (int z = 0; z < batch; ++z) {
             const long long o = (long long)n * z;
             const int m = sytrd_upper(s, n, A + z * sA, k.D + o, k.E + o, k.TAU + o, k.trd, 32,
-                                      vectors ? k.orm + z * sW : nullptr, !whole);
+                                      vectors ? k.orm + z * sW : nullptr, &resident);
             prepare(z, 1, m);
         }
         if (tev) QK_HIP(hipEventRecord(tev[1], s));

@@ -42,7 +42,10 @@
 // About 45 % of a column is the wait for the others' y.
 //
 // Waits end: a reader that sees no progress for SPIN_TICKS raises *fail, which
-// the other workgroups read, and all leave; the caller then runs sytrd_upper.
+// the other workgroups read, and all leave; the caller then runs sytrd_upper, and its
+// owner's later solves do so at once (Resident).  A launch takes 25 ms at most, but its
+// workgroups may come late by the length of whatever kernel another stream of the
+// process has on the device (0.7 s: the densities of 600 orbitals in FP64).
 // Launches whose workgroups wait for each other are kept one after another on
 // the device (resident_gate), each with no more workgroups than it holds.
 #include <mutex>
@@ -561,6 +564,7 @@ const int* trd_resident_fail(int n, int batch, const double* words) {
     return reinterpret_cast<const int*>(words + trd_resident_words(n, batch) - 1);
 }
 bool trd_resident_fits(int n) { return n >= 1 && n <= trd_resident_max() && trd_shape(n, 1) != nullptr; }
+bool trd_resident_waits(int n, int batch) { return n > trd_shape(n, batch)->rows; }
 
 bool trd_resident(hipStream_t s, int n, const double* A, long long lda, long long sA, double* V, long long ldv,
                   long long sV, double* D, double* E, double* TAU, long long sd, int batch, double* words) {

@@ -34,7 +34,8 @@ EXPORTS = ["qk_gw_create", "qk_gw_destroy", "qk_gw_last_error", "qk_gw_set_eri_a
            "qk_rgw_phbse", "qk_gw_sigma_full", "qk_ug0w0", "qk_evugw", "qk_rhf_create", "qk_rhf_destroy", "qk_rhf_last_error", "qk_rhf_set_eri_ao", "qk_rhf_jk", "qk_rhf_jk_ms",
            "qk_rgw_qp_graph_noalloc", "qk_noalloc_last_error", "qk_gw_qp_iters",
            "qk_set_unrestricted_eigensolver", "qk_unrestricted_eig_stats", "qk_gwb_set_graphs", "qk_gwb_graph_stats", "qk_set_split_aotomo",
-           "qk_qsgw_create", "qk_qsgw_cycle", "qk_qsgw_destroy", "qk_qsgw_last_error", "qk_rgw_phbse_dyn", "qk_set_library_gemm", "qk_ugw_phbse"]
+           "qk_qsgw_create", "qk_qsgw_cycle", "qk_qsgw_destroy", "qk_qsgw_last_error", "qk_rgw_phbse_dyn", "qk_set_library_gemm", "qk_ugw_phbse",
+           "qk_gw_set_shared_device", "qk_gwb_set_shared_device"]
 
 
 EIG_MODES = {"syevd": 0, "refine": 1, "sytrd": 2, "refine+sytrd": 3}
@@ -145,6 +146,8 @@ def load():
                              _IP]
     lib.qk_set_unrestricted_eigensolver.argtypes = [_I, _D]
     lib.qk_gwb_set_graphs.argtypes = [_H, _I]
+    lib.qk_gw_set_shared_device.argtypes = [_H, _I]
+    lib.qk_gwb_set_shared_device.argtypes = [_H, _I]
     lib.qk_set_split_aotomo.argtypes = [_I]
     lib.qk_gwb_graph_stats.argtypes = [_H, ctypes.POINTER(ctypes.c_longlong), _I]
     lib.qk_unrestricted_eig_stats.argtypes = [ctypes.POINTER(ctypes.c_longlong), _I]
@@ -233,6 +236,11 @@ class GWEngine:
         Ha, a full solve otherwise; "sytrd" (2), "refine+sytrd" (3): the same
         with the library's own tridiagonalisation in every full solve."""
         _check(load().qk_gw_set_eigensolver(self.h, EIG_MODES.get(mode, mode), de_max), self.h)
+
+    def set_shared_device(self, mode):
+        """1: other processes use this GPU too, so no solve waits inside a launch
+        (qk_gw_set_shared_device); 0: the default; 2: the next such wait counts as failed."""
+        _check(load().qk_gw_set_shared_device(self.h, int(mode)), self.h)
 
     def eig_stats(self):
         c = (ctypes.c_longlong * 9)()
@@ -405,6 +413,10 @@ class GWBatch:
     def set_graphs(self, on):
         """hipGraph replay of evgw()'s cycles from the second cycle of a call."""
         self._check(load().qk_gwb_set_graphs(self.h, int(bool(on))))
+
+    def set_shared_device(self, mode):
+        """As GWEngine.set_shared_device."""
+        self._check(load().qk_gwb_set_shared_device(self.h, int(mode)))
 
     def graph_stats(self):
         c = (ctypes.c_longlong * 2)()
