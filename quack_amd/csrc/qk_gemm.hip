@@ -174,9 +174,11 @@ void launch(hipStream_t s, int M, int N, int K, double alpha, const double* A, l
 }
 
 // Tile configurations: 0: 256 x 32, 1: 64 x 64, 2: 128 x 64, 3: 128 x 128;
-// 4: the library's rocblas_dgemm (only where lib_ok allows it); 5: 32 x 32 (not tuned).
+// 4: the library's rocblas_dgemm (only where lib_ok allows it); 5: 32 x 32 (not tuned, but
+// kept for a shape none of whose trials could be timed).
 constexpr int NOWN = 4, CFG_LIB = 4, CFG_SMALL = 5, NCFG = 5;
-const char* const CFG_NAME[NCFG] = {"256x32", "64x64", "128x64", "128x128", "rocblas"};
+const char* const CFG_NAME[] = {"256x32", "64x64", "128x64", "128x128", "rocblas", "32x32"};
+static_assert(CFG_SMALL < (int)(sizeof CFG_NAME / sizeof *CFG_NAME), "every configuration has a name");
 
 // Library FP64 GEMM as a tuning candidate (qk_set_library_gemm, off by
 // default): plain products only (one matrix, all tiles), 32-bit indexable,
