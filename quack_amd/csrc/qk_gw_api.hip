@@ -1081,10 +1081,10 @@ void after_eri(Ctx* c, bool k_done = false) {
 }
 
 RowUpload::RowUpload(hipStream_t s_, size_t longest, size_t total)
-    : s(s_), slot(std::min(std::max(longest, (size_t)1 << 16), total)) {
+    : s(s_), slot(total <= RING ? total : std::max(longest, RING / SLOTS)), slots(total <= RING ? 1 : SLOTS) {
     try {
-        QK_HIP(hipHostMalloc((void**)&h, SLOTS * slot * sizeof(double), hipHostMallocDefault));
-        for (hipEvent_t& e : ev) QK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        QK_HIP(hipHostMalloc((void**)&h, slots * slot * sizeof(double), hipHostMallocDefault));
+        for (size_t k = 0; slots > 1 && k < slots; ++k) QK_HIP(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
     } catch (...) {
         release();
         throw;
@@ -1099,9 +1099,9 @@ void RowUpload::release() {
 }
 
 void RowUpload::send(double* dst, size_t cnt) {
-    QK_HIP(hipMemcpyAsync(dst, h + turn % SLOTS * slot, cnt * sizeof(double), hipMemcpyHostToDevice, s));
-    QK_HIP(hipEventRecord(ev[turn % SLOTS], s));
-    if (++turn >= SLOTS) QK_HIP(hipEventSynchronize(ev[turn % SLOTS]));
+    QK_HIP(hipMemcpyAsync(dst, h + turn % slots * slot, cnt * sizeof(double), hipMemcpyHostToDevice, s));
+    if (slots > 1) QK_HIP(hipEventRecord(ev[turn % slots], s));
+    ++turn;
 }
 
 void RowUpload::rows(double* dX, const double* base, size_t len, size_t n1, size_t s1, size_t n2, size_t s2, size_t n3,
@@ -1130,7 +1130,8 @@ void RowUpload::rows(double* dX, const double* base, size_t len, size_t n1, size
     };
     for (size_t k = 0; k < 2 + 256 / len; ++k) fetch();
     while (at.i3 < n3) {
-        double* d = h + turn % SLOTS * slot;
+        if (turn >= slots) QK_HIP(slots > 1 ? hipEventSynchronize(ev[turn % slots]) : hipStreamSynchronize(s));
+        double* d = h + turn % slots * slot;
         size_t fill = 0;
         for (; fill < per && at.i3 < n3; ++fill, d += len, at.step()) {
             fetch();

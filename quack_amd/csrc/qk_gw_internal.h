@@ -221,14 +221,20 @@ AoScratch ao_scratch(int N, int n, int nC, int nO, int nR, int nS, double*& buf,
 // array that is in no cache (2.9 KB every 29 KB at N = 60), and a plain copy waits for each
 // row's first lines: 3.6 ms for the 9.3 MB of one block.  The lines of a row some 2 KB of
 // data ahead are asked for while a row is copied, and the copies leave from a short ring of
-// pinned slots while the next one fills (pinning a whole block costs 36 us a megabyte).
+// pinned slots while the next one fills (pinned as a whole, 72 MB took 31 ms).  Every slot
+// sent costs some 10 us of calls, and pinning more than 1.5 MB a call 0.7 ms a megabyte in
+// a program that allocates between calls (phBSE at N = 60: 6.4 ms with two slots of 0.75 MB,
+// 7.4 of 1 MB, 8.9 of 2 MB).  Two slots of 0.75 MB, three of 0.5, and the whole block pinned:
+// 1.7 MB that are in no cache 0.40, 0.57 and 0.42 ms, 9.3 MB 0.86, 1.00 and 1.12; in the
+// caches 0.17, 0.23 and 0.16, 0.53, 0.65 and 0.49.
 struct RowUpload {
-    static constexpr int SLOTS = 3;
+    static constexpr size_t SLOTS = 2, RING = (size_t)3 << 16;  // RING: doubles in all
     hipStream_t s;
-    size_t slot, turn = 0;  // doubles a slot; slots sent
+    size_t slot, slots, turn = 0;  // doubles a slot, slots in the ring, slots sent
     double* h = nullptr;
-    hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr};
-    // for rows of up to `longest` values and calls of up to `total` values
+    hipEvent_t ev[SLOTS] = {};
+    // for rows of up to `longest` values and calls of up to `total` values, which one slot
+    // takes as a whole up to RING
     RowUpload(hipStream_t s_, size_t longest, size_t total);
     RowUpload(const RowUpload&) = delete;
     RowUpload& operator=(const RowUpload&) = delete;
