@@ -357,8 +357,7 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
     if (tid == 0) quit = 0;
     lds_barrier();
     unsigned spins = 0;
-    const int last = g == 0 ? 1 : g + 1;  // the last column this workgroup has a row in
-    for (; c >= last; --c) {
+    for (; c >= 1; --c) {
         const int par = c & 1;
         // row c-1, brought up to date, goes to everyone first: it is on its way while the
         // reflector and y are worked out
@@ -421,7 +420,10 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
             E[c - 1] = h.beta;
             TAU[c - 1] = h.tau;
         }
-        if (g > 0 && c == last) return;
+        // This workgroup's last rows are out.  It goes at the next return, after one look at
+        // words that may be gone: a return here, or another bound of the loop, costs 34
+        // registers (order 3072: 219 spilled instead of 54, 65 ms instead of 23).
+        const bool leave = g > 0 && c <= g + 1;
         double y[KC], dot = 0.0;
         {
             long long t0 = 0;
@@ -442,7 +444,7 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
                     y[k] = 0.0;
                     if (tid + NT * k < c) all = arrived(w + 2 * NT * k, c, y[k]) && all;
                 }
-                if (all && row) break;
+                if ((all && row) || leave) break;
                 if (give_up(spins, t0, p.fail)) {
                     quit = 1;
                     break;
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(NT) void k_trd_wide(TrdArgs p) {
         dot = wave_sum(dot);
         if (lane == 0) red1[q] = dot;
         lds_barrier();
-        if (quit) return;
+        if (quit || leave) return;
         dot = tree_sum<NT / 64>(red1, 1);
         const double half = -0.5 * h.tau * h.tau * dot;
         const double wl = h.tau * ylast + half;  // w(c-1), v(c-1) = 1
