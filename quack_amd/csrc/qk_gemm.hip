@@ -239,7 +239,7 @@ void launch_cfg(int cfg, hipStream_t s, int M, int N, int K, double alpha, const
 // gives every compute unit a workgroup, else the smallest.  One workgroup passes its slabs
 // one after the other, and a slab of a 128 x 128 tile is 64 matrix instructions a wave
 // (1.7 us with one wave a SIMD), of a 32 x 32 tile 4.  128 x 128 and now, us: 225^3 46 and
-// 14, 324^3 61 and 17, 474^3 83 and 24, 225 x 2812 x 225 48 and 21, 95^3 23 and 9.
+// 10, 324^3 61 and 13, 474^3 83 and 18, 225 x 2812 x 225 48 and 18, 95^3 23 and 6.
 int default_cfg(int M, int N, int count) {
     const auto tiles = [&](int b) { return (long long)((M + b - 1) / b) * ((N + b - 1) / b) * count; };
     if (N <= 32 && tiles(32) >= 2048) return 0;

@@ -599,7 +599,8 @@ void screening(Ctx* c, const double* e, const double* eh, int tda, bool vectors)
             // Eigenvectors that go into a split-precision contraction keep the solver they
             // had: the slices round by the vectors' last bits and signs, which differ from
             // solver to solver (2e-11 of a self-energy on the H50 lattice), and evGW's DIIS
-            // makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.
+            // makes 1e-7 Ha of that, where FP64 contractions leave 1e-15.  (Neither solver's
+            // bits are nearer to FP64: 1e-7 Ha is the two-slice form's own error.)
             // qsGW keeps it too: its cycle can amplify the last bits of the vectors without
             // bound where it does not converge (of 24 starts of a compressed H4 chain that
             // differ by 1e-14, 8 converge within 64 cycles and 16 end anywhere), so its

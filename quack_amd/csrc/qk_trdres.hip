@@ -37,8 +37,8 @@
 // row c-1 goes out before the reflector is worked out, and only y is polled for once the
 // row is there (5.1 -> 4.4 and 3.4 -> 2.9); 16 rows a workgroup instead of 32, no
 // branch between the rows of a group.
-// Measured per column: 1.1 us at n = 64, 1.6 at 128, 1.9 at 225, 2.3 at 324, 3.3 at 900,
-// 3.6 at 1326, 4.2 at 2025, 7.4 at 3072; 24 matrices of 324 take 1.05 ms, one 0.74.
+// Measured per column: 1.5 us at n = 95, 1.6 at 128, 2.1 at 225, 2.4 at 324, 3.3 at 900,
+// 3.7 at 1326, 4.1 at 2025, 5.2 at 2500, 7.3 at 3025; 24 matrices of 324 take 1.05 ms, one 0.77.
 // About 45 % of a column is the wait for the others' y.
 //
 // Waits end: a reader that sees no progress for SPIN_TICKS raises *fail, which
